@@ -3,20 +3,23 @@
 // One 256-lane workgroup per 16x16 tile, one lane per pixel.  The tile's depth-sorted
 // entries are staged through LDS in batches (record gather + per-tile pixel rectangle,
 // TileGauss::new at src/rasterize.rs:149-182); every lane walks the batch with its own
-// compositing state, exactly the per-pixel walk of the reference's entry-outer loops.
+// compositing state, exactly the per-pixel walk of the reference's entry-outer loops.  Each
+// 16-lane row of a wave (a 4x4 pixel block) walks its own list of the entries that reach it.
 // The forward pass stops a workgroup when all its pixels are done.
 //
 // Backward: each entry's 11 per-pixel terms are reduced over the tile's pixels and
 // written to the entry's slots (src/rasterize.rs:449-454); a second kernel sums each
-// Gaussian's slots in entry order (src/rasterize.rs:480-503).  ORDERED=true sums the
+// Gaussian's slots in entry order (src/rasterize.rs:480-503).  The ordered kernel sums the
 // pixel terms sequentially in row-major order -- the reference's order, so slots and
-// gradients are bitwise identical to it; ORDERED=false uses DPP row reductions.
+// gradients are bitwise identical to it; the tree-reduced kernel sums each row's pixels by
+// DPP.
 #include "internal.hpp"
 
 namespace splat {
 namespace {
 
-constexpr int kOrdBatch = 8;     // entries per batch (ordered backward)
+constexpr int kOrdBatch = 32;      // entries staged per batch (ordered backward)
+constexpr uint32_t kOrdTerms = 1024;  // pixel terms per slot staged at a time (a tile has 256)
 
 struct TileInfo {
   uint32_t gx0, gy0, w, h;
@@ -112,14 +115,16 @@ __device__ __forceinline__ void clip_range(float m, float half, uint32_t offset,
   *hi_out = as_u32(rclamp(hi, 0.0f, (float)n));
 }
 
-// Packed tile-local rectangle x0 | x1 << 8 | y0 << 16 | y1 << 24 (all <= 16).
+// Tile-local pixel rectangle of an entry as two masks: columns in bits 0-15, rows in bits
+// 16-31 (0: empty).
 __device__ __forceinline__ uint32_t entry_rect(float4 r0, float4 r1, float4 r2, const TileInfo& t) {
   const float hx = r1.w, hy = r2.x;
   if (!(hx >= 0.0f)) return 0u;  // sigma_max <= 0 or det <= 0: empty
-  uint32_t x0, x1, y0, y1;
+  uint32_t x0, x1, y0, y1;  // all <= 16
   clip_range(r0.x, hx, t.gx0, t.w, &x0, &x1);
   clip_range(r0.y, hy, t.gy0, t.h, &y0, &y1);
-  return x0 | (x1 << 8) | (y0 << 16) | (y1 << 24);
+  if (x0 >= x1 || y0 >= y1) return 0u;
+  return ((1u << x1) - (1u << x0)) | (((1u << y1) - (1u << y0)) << 16);
 }
 
 // The records as staged in LDS: conic A (r0.z) and C (r1.x) halved.  Scaling by 1/2
@@ -149,46 +154,37 @@ __device__ __forceinline__ void tile_pixel(uint32_t t, uint32_t* i, uint32_t* j)
   *j = (w >> 1) * 8u + (r >> 1) * 4u + (q >> 2);
 }
 
-// Whether a packed rectangle has pixels in the 4x4 sub-block of row r of wave w.
-__device__ __forceinline__ bool row_touches(uint32_t rc, uint32_t w, uint32_t r) {
-  const uint32_t x0 = rc & 0xffu, x1 = (rc >> 8) & 0xffu, y0 = (rc >> 16) & 0xffu, y1 = rc >> 24;
-  const uint32_t bx = (w & 1u) * 8u + (r & 1u) * 4u, by = (w >> 1) * 8u + (r >> 1) * 4u;
-  return (x0 < x1) & (y0 < y1) & (x0 < bx + 4u) & (x1 > bx) & (y0 < by + 4u) & (y1 > by);
+// Pixels of a rectangle in the 4x4 sub-block of row r of wave w, one bit per lane of the row
+// (bit 4 j + i of the sub-block's pixel (i, j)).
+__device__ __forceinline__ uint32_t row_mask(uint32_t rc, uint32_t w, uint32_t r) {
+  const uint32_t x = (rc >> ((w & 1u) * 8u + (r & 1u) * 4u)) & 0xfu;
+  const uint32_t y = (rc >> (16u + (w >> 1) * 8u + (r >> 1) * 4u)) & 0xfu;
+  const uint32_t rows = (y | (y << 3) | (y << 6) | (y << 9)) & 0x1111u;  // bit j of y to bit 4 j
+  return rows * x;
 }
 
-// Whether a packed rectangle has pixels in the 8x8 block of wave w.
+// Whether a rectangle has pixels in the 8x8 block of wave w.
 __device__ __forceinline__ bool wave_touches(uint32_t rc, uint32_t w) {
-  const uint32_t x0 = rc & 0xffu, x1 = (rc >> 8) & 0xffu, y0 = (rc >> 16) & 0xffu, y1 = rc >> 24;
-  const uint32_t bx = (w & 1u) * 8u, by = (w >> 1) * 8u;
-  return (x0 < x1) & (y0 < y1) & (x0 < bx + 8u) & (x1 > bx) & (y0 < by + 8u) & (y1 > by);
+  return ((rc >> ((w & 1u) * 8u)) & 0xffu) != 0 && ((rc >> (16u + (w >> 1) * 8u)) & 0xffu) != 0;
 }
 
 __device__ __forceinline__ bool in_rect(uint32_t rc, uint32_t i, uint32_t j) {
-  // bitwise, not short-circuit: no divergent branches in the compositing loops
-  return (i >= (rc & 0xffu)) & (i < ((rc >> 8) & 0xffu)) & (j >= ((rc >> 16) & 0xffu)) &
-         (j < (rc >> 24));
+  return ((rc >> i) & (rc >> (16u + j)) & 1u) != 0;
 }
 
-// evaluate, src/rasterize.rs:231-244.
-__device__ __forceinline__ bool evaluate(float4 r0, float4 r1, float px, float py,
-                                         const uint64_t* tab, float* gauss, float* alpha) {
-  const float dx = px - r0.x;
-  const float dy = py - r0.y;
-  const float sigma = 0.5f * (r0.z * dx * dx + r1.x * dy * dy) + r0.w * dx * dy;
-  if (sigma < 0.0f || sigma > r1.z) return false;
-  const float G = expf_tab(-sigma, tab);
-  const float og = r1.y * G;
-  if (og < kAlphaMin) return false;
-  *gauss = G;
-  *alpha = rmin(og, kAlphaMax);
-  return true;
+// A row's entry list in LDS holds words {pixel mask of the row's sub-block << 16 | 16 k} for
+// batch entry k: the low half is the entry's byte offset in a float4 array.  Zero is no
+// entry (an entry in a list has a pixel).
+__device__ __forceinline__ float4 at_bytes(const float4* base, uint32_t bytes) {
+  return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(base) + bytes);
 }
 
 // Pair counters of the counting instantiations (COUNT = true), one 64-bit word each.
-// Forward: (entry, wave) visits, visits in which some lane evaluates the Gaussian,
-// evaluated pairs (sigma in [0, sigma_max]: the exponential is computed), passing pairs
-// (alpha >= 1/255 on a pixel still compositing) and composited pairs.  Backward: visits,
-// active visits, evaluated and passing pairs of the reverse walk.
+// Forward: visits (steps of a wave's walk, one entry of each of its rows' lists), visits in
+// which some lane evaluates its Gaussian, evaluated pairs (sigma in [0, sigma_max]: the
+// exponential is computed), passing pairs (alpha >= 1/255 on a pixel still compositing) and
+// composited pairs.  Backward: visits, active visits, evaluated and passing pairs of the
+// reverse walk.
 enum PairCounter : int {
   kFwdVisits, kFwdActive, kFwdEvaluated, kFwdPassing, kFwdComposited,
   kBwdVisits, kBwdActive, kBwdEvaluated, kBwdPassing, kNumPairCounters
@@ -202,6 +198,12 @@ __device__ __forceinline__ void flush_counts(unsigned long long* pairs, int firs
       if (c[q]) atomicAdd(&pairs[first + q], (unsigned long long)c[q]);
 }
 
+// The forward pass is bound by VALU issue, so it is built for few walk steps and few
+// instructions in each: the four 16-lane rows of a wave walk lists of their own (against one
+// walk of the entries that reach the wave's 8x8 block: about a fifth fewer steps), and a list
+// word carries the pixels of the row's sub-block that the entry's rectangle holds, one AND
+// instead of four comparisons.  At 1M Gaussians, 1920x1080: 226 -> 175 us; 10k Gaussians,
+// 256x256: 82 -> 63 us.
 // B: entries per LDS batch; BATCH: tiles of many views (BatchDev); PERSIST: a fixed grid
 // that takes tiles from `counter` until `num_tiles` are done; COUNT: also count pairs
 // into `pairs` (PairCounter).
@@ -214,11 +216,16 @@ __global__ void __launch_bounds__(256) raster_fwd_kernel(
     float* __restrict__ final_t, uint32_t* __restrict__ n_contrib, BatchDev bd,
     uint32_t* __restrict__ counter, unsigned long long* __restrict__ pairs) {
   static_assert(B <= 256, "each of the 256 lanes stages at most one entry of a batch");
+  constexpr int kList = B < 64 ? B : 64;  // entries per list: one ballot covers them
   __shared__ uint64_t tab[32];
   __shared__ float4 s0[B], s1[B], s2[B];
   __shared__ uint32_t srect[B];
+  __shared__ uint32_t slist[16][kList];  // per (wave, row): its entries, front to back
   __shared__ uint32_t s_tile;
   if (threadIdx.x < 32) tab[threadIdx.x] = kExp2Table[threadIdx.x];
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane >> 4;
+  const uint32_t pixel_bit = 0x10000u << (lane & 15u);
+  const uint32_t* my_list = slist[wave * 4 + row];
   for (;;) {
   const uint32_t tile = next_tile<PERSIST>(counter, &s_tile, order, num_tiles);
   if (tile >= num_tiles) break;
@@ -248,48 +255,67 @@ __global__ void __launch_bounds__(256) raster_fwd_kernel(
     __syncthreads();
     // Predicated form of the per-pixel walk (src/rasterize.rs:262-290): every decision of
     // evaluate() and the T_MIN test is a lane predicate; only the exp is skipped when no
-    // lane of the wave needs it.  Each wave (an 8x8 pixel block) walks, in order, only the
-    // entries whose pixel rectangle reaches its block (a ballot over the batch).
-    for (uint32_t c0k = 0; c0k < cnt; c0k += 64) {
-    const uint32_t kl = c0k + (threadIdx.x & 63);
-    uint64_t todo = __ballot(kl < cnt && wave_touches(srect[min(kl, cnt - 1)], threadIdx.x >> 6));
-    while (todo) {
-      const uint32_t k = c0k + (uint32_t)__builtin_ctzll(todo);
-      todo &= todo - 1;
-      const float4 a = s0[k], b = s1[k];
-      const float dx = px - a.x;
-      const float dy = py - a.y;
-      const float sigma = (a.z * dx * dx + b.x * dy * dy) + a.w * dx * dy;  // halved A, C
-      const bool pass1 = (!done) & in_rect(srect[k], i, j) & !((sigma < 0.0f) | (sigma > b.z));
-      if (COUNT) {
-        const uint64_t b1 = __ballot(pass1);
-        pcount[0]++;
-        if (!b1) continue;
-        pcount[1]++;
-        pcount[2] += (uint32_t)__popcll(b1);
-      } else if (!__any(pass1)) {
-        continue;
+    // lane of the wave needs it.  The four rows of a wave walk, side by side and each in
+    // order, the entries whose pixel rectangle reaches the row's 4x4 sub-block.
+    for (uint32_t c0k = 0; c0k < cnt; c0k += kList) {
+      if (!__any(!done)) break;  // uniform: this wave's pixels are finished
+      const uint32_t kl = c0k + min(lane, (uint32_t)kList - 1u);
+      const uint32_t rc = kl < cnt && lane < (uint32_t)kList ? srect[kl] : 0u;
+      uint32_t steps = 0;
+      // the walk of the previous list is over before this one is written: same wave
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+      for (uint32_t r = 0; r < 4; r++) {
+        const uint32_t pm = row_mask(rc, wave, r);
+        const uint64_t m = __ballot(pm != 0);
+        const uint32_t len = (uint32_t)__popcll(m);
+        uint32_t* list = slist[wave * 4 + r];
+        if (pm) list[__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                               __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] =
+            (pm << 16) | (kl << 4);
+        if (lane >= len && lane < (uint32_t)kList) list[lane] = 0u;  // past the end: no entry
+        steps = max(steps, len);
       }
-      const float G = expf_walk_tab(-sigma, tab);  // used where 0 <= sigma <= sigma_max
-      const float og = b.y * G;
-      const bool pass2 = pass1 & !(og < kAlphaMin);
-      const float alpha = rmin(og, kAlphaMax);
-      const float test_t = T * (1.0f - alpha);
-      const bool stop = test_t < kTMin;
-      done = done | (pass2 & stop);
-      const bool comp = pass2 & !stop;
-      if (COUNT) {
-        pcount[3] += (uint32_t)__popcll(__ballot(pass2));
-        pcount[4] += (uint32_t)__popcll(__ballot(comp));
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      uint32_t last = 0xffffffffu;  // byte offset of the last composited entry of this list
+      for (uint32_t t = 0; t < steps; t++) {
+        const uint32_t le = my_list[t], k16 = le & 0xffffu;
+        const float4 a = at_bytes(s0, k16), b = at_bytes(s1, k16);
+        const float dx = px - a.x;
+        const float dy = py - a.y;
+        const float sigma = (a.z * dx * dx + b.x * dy * dy) + a.w * dx * dy;  // halved A, C
+        const bool pass1 =
+            (!done) & ((le & pixel_bit) != 0) & !((sigma < 0.0f) | (sigma > b.z));
+        if (COUNT) {
+          const uint64_t b1 = __ballot(pass1);
+          pcount[0]++;
+          if (!b1) continue;
+          pcount[1]++;
+          pcount[2] += (uint32_t)__popcll(b1);
+        } else if (__builtin_amdgcn_ballot_w64(pass1) == 0) {
+          continue;
+        }
+        const float4 c = at_bytes(s2, k16);
+        const float G = expf_walk_tab(-sigma, tab);  // used where 0 <= sigma <= sigma_max
+        const float og = b.y * G;
+        const bool pass2 = pass1 & !(og < kAlphaMin);
+        const float alpha = rmin(og, kAlphaMax);
+        const float test_t = T * (1.0f - alpha);
+        const bool stop = test_t < kTMin;
+        done = done | (pass2 & stop);
+        const bool comp = pass2 & !stop;
+        if (COUNT) {
+          pcount[3] += (uint32_t)__popcll(__ballot(pass2));
+          pcount[4] += (uint32_t)__popcll(__ballot(comp));
+        }
+        const float w = alpha * T;
+        c0 = comp ? c0 + w * c.y : c0;
+        c1 = comp ? c1 + w * c.z : c1;
+        c2 = comp ? c2 + w * c.w : c2;
+        T = comp ? test_t : T;
+        last = comp ? k16 : last;
       }
-      const float4 c = s2[k];
-      const float w = alpha * T;
-      c0 = comp ? c0 + w * c.y : c0;
-      c1 = comp ? c1 + w * c.z : c1;
-      c2 = comp ? c2 + w * c.w : c2;
-      T = comp ? test_t : T;
-      nc = comp ? b0 - start + k + 1 : nc;
-    }
+      if (last != 0xffffffffu) nc = b0 - start + (last >> 4) + 1;
     }
   }
   if (valid) {
@@ -326,7 +352,7 @@ __device__ __forceinline__ bool pair_terms(PixBack& s, bool act, float4 r0, floa
   const float dy = py - r0.y;
   const float sigma = (r0.z * dx * dx + r1.x * dy * dy) + r0.w * dx * dy;  // halved A, C
   const bool p1 = act & !((sigma < 0.0f) | (sigma > r1.z));
-  if (!__any(p1)) return false;
+  if (__builtin_amdgcn_ballot_w64(p1) == 0) return false;
   const float G = expf_walk_tab(-sigma, tab);  // used where 0 <= sigma <= sigma_max
   const float o = r1.y;
   const float og = o * G;
@@ -371,6 +397,69 @@ __device__ __forceinline__ bool pair_terms(PixBack& s, bool act, float4 r0, floa
   return true;
 }
 
+// v as seen through a DPP control within each 16-lane row (every lane has a source).  The
+// compiler folds the move into the instruction that consumes it.
+template <int CTRL>
+__device__ __forceinline__ float dpp_row(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+// Sum over each 16-lane row by a rotate butterfly: every lane ends with its row's sum.
+__device__ __forceinline__ float row_allsum16(float v) {
+  v += dpp_row<0x121>(v);  // row_ror:1
+  v += dpp_row<0x122>(v);  // row_ror:2
+  v += dpp_row<0x124>(v);  // row_ror:4
+  v += dpp_row<0x128>(v);  // row_ror:8
+  return v;
+}
+
+// Sums of nine values over each 16-lane row: lanes 2m and 2m+1 of the row end with the sum
+// of v[m] for m < 8, except that lane 15 ends with the sum of v[8].  v[0..7] go through a
+// reduce-scatter whose steps pair a lane with lane ^ {8, 7, 2, 1}; the two partners keep
+// complementary halves of their values (chosen by bit 3, 2, 1 of the lane) and add the half
+// the other sends.  The four masks span all 16 lanes, so every sum covers the row; the order
+// of the additions is fixed.  v[8] goes through row_allsum16's butterfly.
+//
+// The first two steps select by lane bits 3 and 2, which are exactly the DPP banks (lanes
+// 4k .. 4k + 3 of a row): two bank-masked DPP adds, each writing half of the row, give
+// x + x(partner) on one half and y + y(partner) on the other.  The compiler does not form
+// masked DPP adds, so the whole reduction is written out.  A DPP read needs two wait states
+// after the VALU write of its source: v[8]'s steps stand between the others' for that, and
+// two s_nops cover the inputs and the last step (six blocks with a pair of s_nops each spent
+// 12 more issue slots per step of the walk).
+// upper: mask of the lanes with bit 1 set; last: of the rows' lanes 15.
+__device__ __forceinline__ float row_sums9(float v0, float v1, float v2, float v3, float v4,
+                                           float v5, float v6, float v7, float v8,
+                                           uint64_t upper, uint64_t last) {
+  asm volatile(
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"  // banks 0-1: v0
+      "v_add_f32_dpp %0, %4, %4 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"  // banks 2-3: v4
+      "v_add_f32_dpp %1, %1, %1 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %1, %5, %5 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %2, %2, %2 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %2, %6, %6 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %3, %3, %3 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
+      "v_add_f32_dpp %3, %7, %7 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %8, %8, %8 row_ror:1 row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %0, %2, %2 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %8, %8, %8 row_ror:2 row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %1, %1, %1 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
+      "v_add_f32_dpp %1, %3, %3 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %8, %8, %8 row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_e64 %4, %1, %0, %9\n\t"   // the half to send
+      "v_cndmask_b32_e64 %5, %0, %1, %9\n\t"   // the half to keep
+      "v_add_f32_dpp %8, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %0, %4, %5 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_cndmask_b32_e64 %0, %0, %8, %10"
+      : "+v"(v0), "+v"(v1), "+v"(v2), "+v"(v3), "+v"(v4), "+v"(v5), "+v"(v6), "+v"(v7), "+v"(v8)
+      : "s"(upper), "s"(last));
+  return v0;
+}
+
 // pair_terms in the tree-reduced form, rearranged for fewer instructions.  Equal up to
 // rounding; the decisions (sigma range, alpha_min, alpha_max) are the exact ones, so the
 // walk visits the same pairs as the forward:
@@ -389,12 +478,14 @@ __device__ __forceinline__ bool pair_terms(PixBack& s, bool act, float4 r0, floa
 //    q dx dy, q dy^2; the entry's conic turns the sums into dL/dmean and 0.5 scales the
 //    diagonal conic slots once per entry, when the batch's slots are written;
 //  * products with a zero factor stand in for the per-slot selects.
-// The pixel state uses acc0..2 for A; lc and last_alpha are unused.
+// The pixel state uses acc0..2 for A; lc and last_alpha are unused.  Returns the row sums of
+// the slot terms as row_sums9 leaves them in the lanes (with ABS, slots 9 and 10 in the rows'
+// lanes 13 and 11).
 // COUNT: cnt[0..3] += visit, active visit, evaluated and passing pairs.
 template <bool ABS, bool COUNT = false>
-__device__ __forceinline__ bool pair_terms_fast(PixBack& s, bool act, float4 r0, float4 r1,
-                                                float4 r2, float px, float py,
-                                                const uint64_t* tab, bool bg, float v[kSlots],
+__device__ __forceinline__ float pair_sums_fast(PixBack& s, bool act, float4 r0, float4 r1,
+                                                const float4* r2at, float px, float py,
+                                                const uint64_t* tab, bool bg,
                                                 uint32_t* cnt = nullptr) {
   const float dx = px - r0.x;
   const float dy = py - r0.y;
@@ -403,12 +494,13 @@ __device__ __forceinline__ bool pair_terms_fast(PixBack& s, bool act, float4 r0,
   if (COUNT) {
     const uint64_t b1 = __ballot(p1);
     cnt[0]++;
-    if (!b1) return false;
+    if (!b1) return 0.0f;
     cnt[1]++;
     cnt[2] += (uint32_t)__popcll(b1);
-  } else if (!__any(p1)) {
-    return false;
+  } else if (__builtin_amdgcn_ballot_w64(p1) == 0) {
+    return 0.0f;
   }
+  const float4 r2 = *r2at;
   const float G = expf_walk_tab(-sigma, tab);  // used where 0 <= sigma <= sigma_max
   const float o = r1.y;
   const float og = o * G;
@@ -433,101 +525,63 @@ __device__ __forceinline__ bool pair_terms_fast(PixBack& s, bool act, float4 r0,
   }
   const float q = p3 ? -(o * dalpha) * G : 0.0f;
   const float w = p2 ? alpha * t : 0.0f;
-  const float qdx = q * dx, qdy = q * dy;
-  v[0] = qdx;
-  v[1] = qdy;
-  v[2] = qdx * dx;
-  v[3] = qdx * dy;
-  v[4] = qdy * dy;
-  v[5] = p3 ? G * dalpha : 0.0f;
-  v[6] = w * s.d0;
-  v[7] = w * s.d1;
-  v[8] = w * s.d2;
-  if (ABS) {
-    v[9] = fabsf(fmaf(2.0f * r0.z, qdx, r0.w * qdy));
-    v[10] = fabsf(fmaf(r0.w, qdx, (2.0f * r1.x) * qdy));
-  } else {
-    v[9] = v[10] = 0.0f;
-  }
   s.t = p2 ? t : s.t;
   s.acc0 = p2 ? fmaf(alpha, e0, s.acc0) : s.acc0;
   s.acc1 = p2 ? fmaf(alpha, e1, s.acc1) : s.acc1;
   s.acc2 = p2 ? fmaf(alpha, e2, s.acc2) : s.acc2;
-  return true;
-}
-
-// The value of lane (l ^ m) within each 16-lane row, by a DPP control whose partner map is
-// that xor: row_ror:8 (m = 8), row_half_mirror (7), quad_perm [2,3,0,1] (2) and
-// [1,0,3,2] (1).  The compiler folds the move into the add that consumes it.
-template <int CTRL>
-__device__ __forceinline__ float dpp_row(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
-}
-constexpr int kDppXor8 = 0x128, kDppXor7 = 0x141, kDppXor2 = 0x4e, kDppXor1 = 0xb1;
-
-// Reduce-scatter of 8 values over each 16-lane row: afterwards lanes 2m and 2m+1 of the row
-// hold the row's sum of v[m].  Each step pairs a lane with lane ^ {8, 7, 2, 1}; the two
-// partners keep complementary halves of their values (chosen by bit 3, 2, 1 of the lane)
-// and add the half the other sends.  The four masks span all 16 lanes, so every sum covers
-// the row; the order of the additions is fixed.
-//
-// The first two steps select by lane bits 3 and 2, which are exactly the DPP banks (lanes
-// 4k .. 4k + 3 of a row): two bank-masked DPP adds, each writing half of the row, give
-// x + x(partner) on one half and y + y(partner) on the other.  The compiler does not form
-// masked DPP adds, so they are written out; the s_nops give the DPP source reads the wait
-// states they need after the VALU writes around the block.
-__device__ __forceinline__ float dpp_halves_xor8(float x, float y) {  // banks 0-1: x, 2-3: y
-  float out;
-  asm volatile(
-      "s_nop 1\n\t"
-      "v_add_f32_dpp %0, %1, %1 row_ror:8 row_mask:0xf bank_mask:0x3\n\t"
-      "v_add_f32_dpp %0, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-      "s_nop 1"
-      : "=&v"(out)
-      : "v"(x), "v"(y));
-  return out;
-}
-__device__ __forceinline__ float dpp_halves_xor7(float x, float y) {  // banks 0, 2: x; 1, 3: y
-  float out;
-  asm volatile(
-      "s_nop 1\n\t"
-      "v_add_f32_dpp %0, %1, %1 row_half_mirror row_mask:0xf bank_mask:0x5\n\t"
-      "v_add_f32_dpp %0, %2, %2 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
-      "s_nop 1"
-      : "=&v"(out)
-      : "v"(x), "v"(y));
+  const float qdx = q * dx, qdy = q * dy;
+  constexpr uint64_t kUpper = 0xccccccccccccccccull, kLast = 0x8000800080008000ull;
+  float out = row_sums9(qdx, qdy, qdx * dx, qdx * dy, qdy * dy, p3 ? G * dalpha : 0.0f, w * s.d0,
+                        w * s.d1, w * s.d2, kUpper, kLast);
+  if (ABS) {
+    const float e9 = row_allsum16(fabsf(fmaf(2.0f * r0.z, qdx, r0.w * qdy)));
+    const float e10 = row_allsum16(fabsf(fmaf(r0.w, qdx, (2.0f * r1.x) * qdy)));
+    const uint32_t l16 = threadIdx.x & 15u;
+    out = l16 == 13 ? e9 : out;
+    out = l16 == 11 ? e10 : out;
+  }
   return out;
 }
 
-__device__ __forceinline__ float row_scatter8(const float v[8], uint32_t lane) {
-  const bool b1 = (lane & 2u) != 0;
-  float a[4], b[2];
-#pragma unroll
-  for (int q = 0; q < 4; q++) a[q] = dpp_halves_xor8(v[q], v[q + 4]);
-#pragma unroll
-  for (int q = 0; q < 2; q++) b[q] = dpp_halves_xor7(a[q], a[q + 2]);
-  const float c = (b1 ? b[1] : b[0]) + dpp_row<kDppXor2>(b1 ? b[0] : b[1]);
-  return c + dpp_row<kDppXor1>(c);
+// A pixel's state at the start of the backward walk.  valid: inside the image.
+__device__ __forceinline__ PixBack pixel_back(const TileGeom& tg, uint32_t i, uint32_t j,
+                                              bool valid, float bg0, float bg1, float bg2,
+                                              const float* __restrict__ final_t,
+                                              const uint32_t* __restrict__ n_contrib,
+                                              const float* __restrict__ dimage) {
+  PixBack s;
+  s.acc0 = s.acc1 = s.acc2 = 0.0f;
+  s.lc0 = s.lc1 = s.lc2 = 0.0f;
+  s.last_alpha = 0.0f;
+  s.t = 1.0f;
+  s.t_final = 1.0f;
+  s.d0 = s.d1 = s.d2 = 0.0f;
+  s.bg_dot = 0.0f;
+  s.last = 0;
+  if (valid) {
+    const size_t pix = tg.pix0 + (size_t)(tg.ti.gy0 + j) * tg.width + tg.ti.gx0 + i;
+    s.d0 = dimage[pix * 3 + 0];
+    s.d1 = dimage[pix * 3 + 1];
+    s.d2 = dimage[pix * 3 + 2];
+    s.bg_dot = bg0 * s.d0 + bg1 * s.d1 + bg2 * s.d2;
+    s.last = n_contrib[pix];
+    s.t_final = final_t[pix];
+    s.t = s.t_final;
+  }
+  return s;
 }
 
-// Sum over each 16-lane row by a rotate butterfly: every lane ends with its row's sum.
-__device__ __forceinline__ float row_allsum16(float v) {
-  v += dpp_row<0x121>(v);  // row_ror:1
-  v += dpp_row<0x122>(v);  // row_ror:2
-  v += dpp_row<0x124>(v);  // row_ror:4
-  v += dpp_row<0x128>(v);  // row_ror:8
-  return v;
-}
-
-// ORDERED: per-pixel terms staged in LDS and summed sequentially in row-major order.
-// Otherwise: 16-lane row sums by DPP, 16 row partials per entry summed in a fixed order.
-// ABS: also accumulate the AbsGS slots (9, 10); otherwise they are written as zero.
-// BF: entries per LDS batch of the tree-reduced form (the ordered form uses kOrdBatch).
-// ROWS (tree-reduced form): every 16-lane row walks its own entry list; otherwise the wave
-// walks the entries that reach any of its rows (the same sums either way).  COUNT
-// (tree-reduced form only): also count pairs into `pairs` (PairCounter).
-template <bool ORDERED, bool ABS, int BF, bool BATCH, bool PERSIST, bool ROWS,
-          bool COUNT = false>
+// The tree-reduced backward: 16-lane row sums by DPP (row_sums9), an entry's row partials
+// summed in a fixed order.  Bound by VALU issue (about 100 instructions per walk step).  Of
+// the LDS partials only those that svisit names are written and read: clearing all 16 rows of
+// every entry and summing them took as many instructions as a fifth of the walk.  With that,
+// the list words (as in the forward) and the row sums in one block: 1M Gaussians, 1920x1080,
+// 471 -> 400 us; 10k, 256x256, 139 -> 123 us.
+// ABS: also accumulate the AbsGS slots (9, 10).  B: entries per LDS batch.  ROWS: every
+// 16-lane row walks its own entry list; otherwise the wave walks the entries that reach any
+// of its rows (the same sums either way).  COUNT: also count pairs into `pairs`
+// (PairCounter).
+template <bool ABS, int B, bool BATCH, bool PERSIST, bool ROWS, bool COUNT = false>
 __global__ void __launch_bounds__(256) raster_bwd_kernel(
     const float4* __restrict__ rec, const uint32_t* __restrict__ tile_start,
     const uint32_t* __restrict__ order,
@@ -536,24 +590,30 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
     float bg2, const float* __restrict__ final_t, const uint32_t* __restrict__ n_contrib,
     const float* __restrict__ dimage, float* __restrict__ slots, BatchDev bd,
     uint32_t* __restrict__ counter, unsigned long long* __restrict__ pairs) {
-  static_assert(!(COUNT && ORDERED), "pairs are counted in the tree-reduced form");
-  constexpr int B = ORDERED ? kOrdBatch : BF;
+  static_assert(B <= 32, "a list is built by half a wave");
+  // words per entry in `slots` and per row partial: the absolute sums (9, 10) only when asked
+  constexpr uint32_t SS = ABS ? kSlots : 9;
   __shared__ uint64_t tab[32];
   __shared__ float4 s0[B], s1[B], s2[B];
   __shared__ uint32_t srect[B];
+  __shared__ __align__(4) uint8_t svisit[B][4];  // per entry and wave: the rows that wrote a partial
+  __shared__ uint32_t slist[16][B];    // per (wave, row): its entries, back to front
   __shared__ uint32_t smax_last;
   __shared__ uint32_t s_tile;
-  // per (wave, row): the batch entries the row walks, back to front
-  __shared__ uint8_t slist[ORDERED ? 1 : 16][ORDERED ? 1 : B];
-  // words per entry in `slots`: the absolute sums (slots 9, 10) only when asked for
-  constexpr uint32_t SS = ABS ? kSlots : 9;
-  // ORDERED: per-pixel terms of the batch; otherwise per-row partial sums of the SS slots
-  // (18 KB at B = 32 without the absolute sums; the workgroup's LDS is then about 20.4 KB,
-  // seven workgroups per CU, as many as its 72 VGPRs allow).
-  __shared__ float red[ORDERED ? B * kSlots * 256 : B * SS * 16];
+  // Partials of the batch, [entry][wave, row][word]; only those named by svisit are written
+  // and read (an entry reaches 2 to 3 of a tile's 16 rows on average).
+  __shared__ float red[B * 16 * SS];
   // whether the background term (T_final bg . dL) can be non-zero for a finite dL
   const bool bg_any = (bg0 != 0.0f) | (bg1 != 0.0f) | (bg2 != 0.0f);
   if (threadIdx.x < 32) tab[threadIdx.x] = kExp2Table[threadIdx.x];
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane >> 4;
+  const uint32_t l16 = lane & 15u;
+  const uint32_t pixel_bit = 0x10000u << l16;
+  // the slot whose row sum this lane holds after a step, if it writes one: even lane 2m slot
+  // m, lane 15 slot 8, lanes 13 and 11 the AbsGS slots 9 and 10
+  const bool even = (l16 & 1u) == 0;
+  const bool writer = even | (l16 == 15) | (ABS & ((l16 == 13) | (l16 == 11)));
+  const uint32_t wslot = even ? (l16 >> 1) : (l16 == 15 ? 8u : (l16 == 13 ? 9u : 10u));
   for (;;) {
   const uint32_t tile = next_tile<PERSIST>(counter, &s_tile, order, num_tiles);
   if (tile >= num_tiles) break;
@@ -565,25 +625,7 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
   const bool valid = i < ti.w && j < ti.h;
   const float px = (float)(ti.gx0 + i) + 0.5f;
   const float py = (float)(ti.gy0 + j) + 0.5f;
-  PixBack s;
-  s.acc0 = s.acc1 = s.acc2 = 0.0f;
-  s.lc0 = s.lc1 = s.lc2 = 0.0f;
-  s.last_alpha = 0.0f;
-  s.t = 1.0f;
-  s.t_final = 1.0f;
-  s.d0 = s.d1 = s.d2 = 0.0f;
-  s.bg_dot = 0.0f;
-  s.last = 0;
-  if (valid) {
-    const size_t pix = tg.pix0 + (size_t)(ti.gy0 + j) * tg.width + ti.gx0 + i;
-    s.d0 = dimage[pix * 3 + 0];
-    s.d1 = dimage[pix * 3 + 1];
-    s.d2 = dimage[pix * 3 + 2];
-    s.bg_dot = bg0 * s.d0 + bg1 * s.d1 + bg2 * s.d2;
-    s.last = n_contrib[pix];
-    s.t_final = final_t[pix];
-    s.t = s.t_final;
-  }
+  PixBack s = pixel_back(tg, i, j, valid, bg0, bg1, bg2, final_t, n_contrib, dimage);
   const uint32_t start = tile_start[tile], end = tile_start[tile + 1];
   const uint32_t count = end - start;
   uint32_t pcount[4] = {0, 0, 0, 0};
@@ -596,7 +638,6 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
     const uint32_t k = q / SS;
     slots[(size_t)sorted_entry[start + k] * SS + q % SS] = 0.0f;
   }
-  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane >> 4;
   // the last contributor of any pixel of each 16-lane row of this wave
   uint32_t row_last[4];
   {
@@ -606,6 +647,7 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
 #pragma unroll
     for (int r = 0; r < 4; r++) row_last[r] = (uint32_t)__builtin_amdgcn_readlane((int)m, 16 * r);
   }
+  const uint32_t wave_last = max(max(row_last[0], row_last[1]), max(row_last[2], row_last[3]));
   // Batches walk [0, kmax) from the back.
   for (int32_t hi = (int32_t)kmax; hi > 0; hi -= B) {
     const int32_t lo = max(hi - B, 0);
@@ -619,115 +661,205 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
       s2[threadIdx.x] = c;
       srect[threadIdx.x] = entry_rect(a, b, c, ti);
     }
-    if (!ORDERED)  // partials of entries a wave skips stay zero
-      for (uint32_t q = threadIdx.x; q < cnt * SS * 16; q += blockDim.x) red[q] = 0.0f;
     __syncthreads();
-    if (ORDERED) {
-      for (int32_t kk = (int32_t)cnt - 1; kk >= 0; kk--) {
-        const uint32_t k = lo + kk;
-        float v[kSlots];
-        const bool act = valid & (k < s.last) & in_rect(srect[kk], i, j);
-        pair_terms(s, act, s0[kk], s1[kk], s2[kk], px, py, tab, v);
+    // Each 16-lane row walks, back to front, only the batch entries that reach its 4x4
+    // sub-block and precede the row's last contributor; the four rows of a wave walk
+    // their own lists side by side.  Lanes 0-31 build the lists of rows 0 and 1, lanes
+    // 32-63 those of rows 2 and 3, one entry per lane.
+    const uint32_t kl = lane & 31u, half = lane >> 5;
+    const uint32_t rc = kl < cnt ? srect[min(kl, (uint32_t)B - 1u)] : 0u;
+    uint32_t steps = 0, visit = 0;
+    uint64_t wave_todo = 0;  // !ROWS: the wave's entries, walked from the top bit down
+    if (ROWS) {
 #pragma unroll
-        for (int q = 0; q < kSlots; q++) red[(kk * kSlots + q) * 256 + j * kTile + i] = v[q];
+      for (uint32_t r = 0; r < 2; r++) {
+        const uint32_t last = half ? row_last[r + 2] : row_last[r];
+        const uint32_t pm = lo + kl < last ? row_mask(rc, wave, half * 2 + r) : 0u;
+        const uint64_t m2 = __ballot(pm != 0);
+        const uint32_t lo_half = (uint32_t)m2, hi_half = (uint32_t)(m2 >> 32);
+        const uint32_t m = half ? hi_half : lo_half;
+        const uint32_t len = (uint32_t)__popc(m);
+        uint32_t* list = slist[wave * 4 + half * 2 + r];
+        // entry kl sits behind the later entries of the batch
+        if (pm) list[__popc(m >> kl) - 1] = (pm << 16) | (kl << 4);
+        if (kl >= len && kl < (uint32_t)B) list[kl] = 0u;  // past the end: no entry
+        if (pm) visit |= 1u << r;
+        steps = max(steps, max((uint32_t)__popc(lo_half), (uint32_t)__popc(hi_half)));
       }
+      visit |= (uint32_t)__shfl((int)visit, (int)(kl + 32), 64) << 2;  // for lanes 0-31
     } else {
-      // Each 16-lane row walks, back to front, only the batch entries that reach its 4x4
-      // sub-block and precede the row's last contributor; the four rows of a wave walk
-      // their own lists side by side (B <= 64: one ballot per row covers the batch).
-      // Sums over each 16-lane row: slots 0-7 by one reduce-scatter (even lane 2m holds
-      // slot m), slot 8 (and the AbsGS slots 9, 10) by a butterfly read from lane 15 (13,
-      // 11); one LDS store per writer lane.
-      const uint32_t l16 = lane & 15u;
-      const bool even = (l16 & 1u) == 0;
-      const bool writer = even | (l16 == 15) | (ABS & ((l16 == 13) | (l16 == 11)));
-      const uint32_t wslot = even ? (l16 >> 1) : (l16 == 15 ? 8u : (l16 == 13 ? 9u : 10u));
-      const uint32_t woff = wslot * 16 + wave * 4 + row;
-      // the rows' lists: entry kk sits at position popcount(mask >> (kk + 1))
-      uint8_t* my_list = slist[wave * 4 + row];
-      const uint32_t kl = min(lane, cnt - 1);
-      uint32_t steps = 0, my_len = 0;
-      uint64_t wave_todo = 0;  // !ROWS: the wave's entries, walked from the top bit down
+      const bool on = lane < cnt && lo + lane < wave_last && wave_touches(rc, wave);
+      wave_todo = __ballot(on);
+      steps = (uint32_t)__popcll(wave_todo);
+      visit = on ? 0xfu : 0u;
+    }
+    if (lane < cnt) svisit[lane][wave] = (uint8_t)visit;
+    // the lists are written and read by this wave only
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    const uint32_t* my_list = slist[wave * 4 + row];
+    const uint32_t last16 = s.last > (uint32_t)lo ? min(s.last - lo, (uint32_t)B) << 4 : 0u;
+    for (uint32_t t = 0; t < steps; t++) {
+      uint32_t k16;
+      bool has = true, act;
       if (ROWS) {
-        uint32_t len[4];
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const uint64_t m = __ballot(lane < cnt && lo + lane < row_last[r] &&
-                                      row_touches(srect[kl], wave, (uint32_t)r));
-          len[r] = (uint32_t)__popcll(m);
-          if ((m >> lane) & 1ull)
-            slist[wave * 4 + r][__popcll(m >> lane) - 1] = (uint8_t)lane;
-        }
-        steps = max(max(len[0], len[1]), max(len[2], len[3]));
-        my_len = row == 0 ? len[0] : (row == 1 ? len[1] : (row == 2 ? len[2] : len[3]));
-        // the lists are written and read by this wave only
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        const uint32_t le = my_list[t];
+        k16 = le & 0xffffu;
+        has = le != 0;
+        act = ((le & pixel_bit) != 0) & (k16 < last16);
       } else {
-        const uint32_t wave_last =
-            max(max(row_last[0], row_last[1]), max(row_last[2], row_last[3]));
-        wave_todo = __ballot(lane < cnt && lo + lane < wave_last &&
-                             wave_touches(srect[kl], wave));
-        steps = (uint32_t)__popcll(wave_todo);
-        my_len = steps;
+        const uint32_t kk = 63u - (uint32_t)__builtin_clzll(wave_todo);
+        wave_todo &= ~(1ull << kk);
+        k16 = kk << 4;
+        act = (k16 < last16) & in_rect(srect[kk], i, j);
       }
-      for (uint32_t t = 0; t < steps; t++) {
-        const bool has = t < my_len;
-        uint32_t kk;
-        if (ROWS) {
-          kk = has ? (uint32_t)my_list[t] : 0u;
-        } else {
-          kk = 63u - (uint32_t)__builtin_clzll(wave_todo);
-          wave_todo &= ~(1ull << kk);
-        }
-        const uint32_t k = lo + kk;
-        float v[kSlots];
-        const bool act = has & valid & (k < s.last) & in_rect(srect[kk], i, j);
-        if (pair_terms_fast<ABS, COUNT>(s, act, s0[kk], s1[kk], s2[kk], px, py, tab, bg_any, v,
-                                        pcount)) {
-          float r = row_scatter8(v, lane);
-          const float e8 = row_allsum16(v[8]);
-          r = l16 == 15 ? e8 : r;
-          if (ABS) {
-            const float e9 = row_allsum16(v[9]);
-            const float e10 = row_allsum16(v[10]);
-            r = l16 == 13 ? e9 : r;
-            r = l16 == 11 ? e10 : r;
-          }
-          if (writer & has) red[kk * SS * 16 + woff] = r;
-        }
-      }
+      const float4* r2at = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(s2) + k16);
+      const float out = pair_sums_fast<ABS, COUNT>(s, act, at_bytes(s0, k16), at_bytes(s1, k16),
+                                                   r2at, px, py, tab, bg_any, pcount);
+      if (has & writer) red[k16 * SS + (wave * 4 + row) * SS + wslot] = out;
     }
     __syncthreads();
-    // Reduce the batch and write its slots.
-    for (uint32_t q = threadIdx.x; q < cnt * SS; q += blockDim.x) {
-      const uint32_t kk = q / SS, slot = q % SS;
-      float acc = 0.0f;
-      if (ORDERED) {
-        const float* p = &red[(kk * kSlots + slot) * 256];
-        for (int t = 0; t < 256; t++) acc += p[t];
-      } else {
-        // pair_terms_fast's products: slots 0, 1 combine both position sums with the conic
-        const auto part_sum = [&](uint32_t sl) {
-          const float* p = &red[(kk * SS + sl) * 16];
-          float a = 0.0f;
-#pragma unroll
-          for (int t = 0; t < 16; t++) a += p[t];
-          return a;
-        };
-        if (slot < 2) {
-          const float sx = part_sum(0), sy = part_sum(1);
-          const float4 a = s0[kk];
-          acc = slot == 0 ? -fmaf(2.0f * a.z, sx, a.w * sy)
-                          : -fmaf(a.w, sx, (2.0f * s1[kk].x) * sy);
-        } else if (ABS || slot < 9) {
-          acc = part_sum(slot);
-          if (slot == 2 || slot == 4) acc *= 0.5f;
+    // Sum the batch's partials and write its slots: 16 lanes per entry, lane = slot.
+    const uint32_t slot = threadIdx.x & 15u;
+    for (uint32_t e0 = 0; e0 < cnt; e0 += 16) {
+      const uint32_t kk = e0 + (threadIdx.x >> 4);
+      if (kk < cnt && slot < SS) {
+        const float4 a = s0[kk], b = s1[kk];
+        const uint32_t v = *reinterpret_cast<const uint32_t*>(svisit[kk]);
+        uint32_t rows =
+            (v & 0xfu) | ((v >> 4) & 0xf0u) | ((v >> 8) & 0xf00u) | ((v >> 12) & 0xf000u);
+        const float* p = &red[kk * 16 * SS + slot];
+        float acc = 0.0f;
+        while (rows) {
+          acc += p[(uint32_t)__builtin_ctz(rows) * SS];
+          rows &= rows - 1;
         }
+        // pair_sums_fast's products: slots 0, 1 combine both position sums with the conic
+        const float other = dpp_row<0xb1>(acc);  // lane ^ 1
+        if (slot == 0)
+          acc = -fmaf(2.0f * a.z, acc, a.w * other);
+        else if (slot == 1)
+          acc = -fmaf(a.w, other, (2.0f * b.x) * acc);
+        else if (slot == 2 || slot == 4)
+          acc *= 0.5f;
+        slots[(size_t)sorted_entry[start + lo + kk] * SS + slot] = acc;
       }
-      slots[(size_t)sorted_entry[start + lo + kk] * SS + slot] = acc;
     }
   }
   if (COUNT) flush_counts(pairs, kBwdVisits, pcount, 4);
+  if (!PERSIST) break;
+  }
+}
+
+// The ordered backward: an entry's per-pixel terms are staged in LDS and summed one by one
+// in row-major order.  Only the pixels of the entry's rectangle have terms (the others are
+// exact zeros, which a sum that starts at +0 does not see), so the staging is packed: the
+// entries of a group, as many as fit kOrdTerms pixels, lie one after the other, and a lane
+// sums one slot of one entry over the entry's own pixels.  Only the waves whose 8x8 block the
+// rectangle reaches evaluate it.
+template <bool ABS, bool BATCH, bool PERSIST>
+__global__ void __launch_bounds__(256) raster_bwd_ordered_kernel(
+    const float4* __restrict__ rec, const uint32_t* __restrict__ tile_start,
+    const uint32_t* __restrict__ order,
+    const uint32_t* __restrict__ sorted_gauss, const uint32_t* __restrict__ sorted_entry,
+    uint32_t num_tiles, uint32_t tiles_x, uint32_t W, uint32_t H, float bg0, float bg1,
+    float bg2, const float* __restrict__ final_t, const uint32_t* __restrict__ n_contrib,
+    const float* __restrict__ dimage, float* __restrict__ slots, BatchDev bd,
+    uint32_t* __restrict__ counter) {
+  constexpr uint32_t SS = ABS ? kSlots : 9;
+  constexpr int B = kOrdBatch;
+  static_assert(B <= 64 && kOrdTerms >= 256, "one wave scans a batch; a group holds an entry");
+  __shared__ uint64_t tab[32];
+  __shared__ float4 s0[B], s1[B], s2[B];
+  __shared__ uint32_t srect[B];
+  __shared__ uint32_t spre[B + 1];  // pixels of the batch entries before each one
+  __shared__ uint32_t smax_last;
+  __shared__ uint32_t s_tile;
+  __shared__ float terms[SS * kOrdTerms];
+  if (threadIdx.x < 32) tab[threadIdx.x] = kExp2Table[threadIdx.x];
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (;;) {
+  const uint32_t tile = next_tile<PERSIST>(counter, &s_tile, order, num_tiles);
+  if (tile >= num_tiles) break;
+  if (threadIdx.x == 0) smax_last = 0;
+  const TileGeom tg = tile_geom<BATCH>(tile, tiles_x, W, H, bd);
+  const TileInfo ti = tg.ti;
+  uint32_t i, j;
+  tile_pixel(threadIdx.x, &i, &j);
+  const bool valid = i < ti.w && j < ti.h;
+  const float px = (float)(ti.gx0 + i) + 0.5f;
+  const float py = (float)(ti.gy0 + j) + 0.5f;
+  PixBack s = pixel_back(tg, i, j, valid, bg0, bg1, bg2, final_t, n_contrib, dimage);
+  const uint32_t start = tile_start[tile], end = tile_start[tile + 1];
+  const uint32_t count = end - start;
+  __syncthreads();
+  if (valid && s.last > 0) atomicMax(&smax_last, s.last);
+  __syncthreads();
+  const uint32_t kmax = min(smax_last, count);
+  // Entries no pixel reaches get zero slots.
+  for (uint32_t q = kmax * SS + threadIdx.x; q < count * SS; q += blockDim.x) {
+    const uint32_t k = q / SS;
+    slots[(size_t)sorted_entry[start + k] * SS + q % SS] = 0.0f;
+  }
+  for (int32_t hi = (int32_t)kmax; hi > 0; hi -= B) {
+    const int32_t lo = max(hi - B, 0);
+    const uint32_t cnt = (uint32_t)(hi - lo);
+    __syncthreads();
+    if (threadIdx.x < 64) {
+      uint32_t area = 0;
+      if (threadIdx.x < cnt) {
+        const uint32_t g = sorted_gauss[start + lo + threadIdx.x];
+        const float4 a = rec[4 * g], b = rec[4 * g + 1], c = rec[4 * g + 2];
+        s0[threadIdx.x] = half_conic0(a);
+        s1[threadIdx.x] = half_conic1(b);
+        s2[threadIdx.x] = c;
+        const uint32_t rc = entry_rect(a, b, c, ti);
+        srect[threadIdx.x] = rc;
+        area = (uint32_t)__popc(rc & 0xffffu) * (uint32_t)__popc(rc >> 16);
+      }
+      uint32_t pre = area;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)pre, d, 64);
+        if (lane >= (uint32_t)d) pre += o;
+      }
+      if (lane <= cnt && lane <= (uint32_t)B) spre[lane] = pre - area;
+    }
+    __syncthreads();
+    // groups of entries from the back, each the longest that fits the staging
+    const uint32_t my_pre = spre[min(lane, cnt)];
+    for (uint32_t g1 = cnt; g1 > 0;) {
+      const uint32_t p1 = spre[g1];
+      const uint64_t fits = __ballot(lane < g1 && p1 - my_pre <= kOrdTerms);
+      const uint32_t g0 = (uint32_t)__builtin_ctzll(fits);  // entry g1 - 1 fits (<= 256 pixels)
+      const uint32_t p0 = spre[g0];
+      uint64_t todo = __ballot(lane >= g0 && lane < g1 && wave_touches(srect[min(lane, cnt - 1)], wave));
+      while (todo) {
+        const uint32_t kk = 63u - (uint32_t)__builtin_clzll(todo);
+        todo &= ~(1ull << kk);
+        const uint32_t rc = srect[kk];
+        const bool in = in_rect(rc, i, j);  // columns and rows are within the image
+        float v[kSlots];
+        pair_terms(s, valid & (lo + kk < s.last) & in, s0[kk], s1[kk], s2[kk], px, py, tab, v);
+        if (in) {
+          const uint32_t x0 = (uint32_t)__builtin_ctz(rc), y0 = (uint32_t)__builtin_ctz(rc >> 16);
+          const uint32_t pos = spre[kk] - p0 + (j - y0) * (uint32_t)__popc(rc & 0xffffu) + (i - x0);
+#pragma unroll
+          for (int q = 0; q < (int)SS; q++) terms[q * kOrdTerms + pos] = v[q];
+        }
+      }
+      __syncthreads();
+      for (uint32_t q = threadIdx.x; q < (g1 - g0) * SS; q += blockDim.x) {
+        const uint32_t kk = g0 + q / SS, slot = q % SS;
+        const uint32_t n = spre[kk + 1] - spre[kk];
+        const float* p = &terms[slot * kOrdTerms + (spre[kk] - p0)];
+        float acc = 0.0f;
+        for (uint32_t t = 0; t < n; t++) acc += p[t];
+        slots[(size_t)sorted_entry[start + lo + kk] * SS + slot] = acc;
+      }
+      __syncthreads();
+      g1 = g0;
+    }
+  }
   if (!PERSIST) break;
   }
 }
@@ -812,19 +944,33 @@ void fwd_go(splat_ctx* ctx, const ProjBuffers& pb, const BinBuffers& bb, unsigne
          image, final_t, n_contrib, bd, counter, (unsigned long long*)nullptr);
 }
 
-template <bool ORDERED, bool ABS, int BF, bool BATCH, bool PERSIST, bool ROWS>
-void bwd_go(splat_ctx* ctx, const char* name, const ProjBuffers& pb, const BinBuffers& bb,
-            unsigned T, uint32_t width, uint32_t height, const float bg[3], const float* final_t,
+template <bool ABS, int BF, bool BATCH, bool PERSIST, bool ROWS>
+void bwd_go(splat_ctx* ctx, const ProjBuffers& pb, const BinBuffers& bb, unsigned T,
+            uint32_t width, uint32_t height, const float bg[3], const float* final_t,
             const uint32_t* n_contrib, const float* dimage, float* slots, const BatchDev& bd,
             uint32_t* counter, unsigned per_cu) {
   if (PERSIST) fill_u32(ctx, counter, kXcds, 0u);
   const unsigned grid = PERSIST ? persistent_grid(ctx, per_cu, T) : T;
-  launch(ctx, name, raster_bwd_kernel<ORDERED, ABS, BF, BATCH, PERSIST, ROWS>, dim3(grid), dim3(256),
-         0, (const float4*)pb.rec, (const uint32_t*)bb.tile_start,
+  launch(ctx, "raster_bwd", raster_bwd_kernel<ABS, BF, BATCH, PERSIST, ROWS>, dim3(grid),
+         dim3(256), 0, (const float4*)pb.rec, (const uint32_t*)bb.tile_start,
          (const uint32_t*)bb.tile_order, (const uint32_t*)bb.sorted_gauss,
          (const uint32_t*)bb.sorted_entry, T, bb.tiles_x, width,
          height, bg[0], bg[1], bg[2], final_t, n_contrib, dimage, slots, bd, counter,
          (unsigned long long*)nullptr);
+}
+
+template <bool ABS, bool BATCH, bool PERSIST>
+void bwd_ordered_go(splat_ctx* ctx, const ProjBuffers& pb, const BinBuffers& bb, unsigned T,
+                    uint32_t width, uint32_t height, const float bg[3], const float* final_t,
+                    const uint32_t* n_contrib, const float* dimage, float* slots,
+                    const BatchDev& bd, uint32_t* counter, unsigned per_cu) {
+  if (PERSIST) fill_u32(ctx, counter, kXcds, 0u);
+  const unsigned grid = PERSIST ? persistent_grid(ctx, per_cu, T) : T;
+  launch(ctx, "raster_bwd_ordered", raster_bwd_ordered_kernel<ABS, BATCH, PERSIST>, dim3(grid),
+         dim3(256), 0, (const float4*)pb.rec, (const uint32_t*)bb.tile_start,
+         (const uint32_t*)bb.tile_order, (const uint32_t*)bb.sorted_gauss,
+         (const uint32_t*)bb.sorted_entry, T, bb.tiles_x, width,
+         height, bg[0], bg[1], bg[2], final_t, n_contrib, dimage, slots, bd, counter);
 }
 
 template <bool BATCH, bool PERSIST>
@@ -857,20 +1003,16 @@ void bwd_rows_pick(splat_ctx* ctx, const RasterVariant& rv, const ProjBuffers& p
   const unsigned pc = rv.per_cu;
   if (rv.bwd_batch == 16) {
     if (need_abs)
-      return bwd_go<false, true, 16, BATCH, PERSIST, ROWS>(ctx, "raster_bwd", pb, bb, T, width,
-                                                           height, bg, final_t, n_contrib,
-                                                           dimage, slots, bd, counter, pc);
-    return bwd_go<false, false, 16, BATCH, PERSIST, ROWS>(ctx, "raster_bwd", pb, bb, T, width,
-                                                          height, bg, final_t, n_contrib, dimage,
-                                                          slots, bd, counter, pc);
+      return bwd_go<true, 16, BATCH, PERSIST, ROWS>(ctx, pb, bb, T, width, height, bg, final_t,
+                                                    n_contrib, dimage, slots, bd, counter, pc);
+    return bwd_go<false, 16, BATCH, PERSIST, ROWS>(ctx, pb, bb, T, width, height, bg, final_t,
+                                                   n_contrib, dimage, slots, bd, counter, pc);
   }
   if (need_abs)
-    return bwd_go<false, true, 32, BATCH, PERSIST, ROWS>(ctx, "raster_bwd", pb, bb, T, width,
-                                                         height, bg, final_t, n_contrib, dimage,
-                                                         slots, bd, counter, pc);
-  return bwd_go<false, false, 32, BATCH, PERSIST, ROWS>(ctx, "raster_bwd", pb, bb, T, width,
-                                                        height, bg, final_t, n_contrib, dimage,
-                                                        slots, bd, counter, pc);
+    return bwd_go<true, 32, BATCH, PERSIST, ROWS>(ctx, pb, bb, T, width, height, bg, final_t,
+                                                  n_contrib, dimage, slots, bd, counter, pc);
+  return bwd_go<false, 32, BATCH, PERSIST, ROWS>(ctx, pb, bb, T, width, height, bg, final_t,
+                                                 n_contrib, dimage, slots, bd, counter, pc);
 }
 
 template <bool BATCH, bool PERSIST>
@@ -882,13 +1024,11 @@ void bwd_pick(splat_ctx* ctx, const RasterVariant& rv, const ProjBuffers& pb,
   const unsigned pc = rv.per_cu;
   // the record width (9 or 11 words per entry) follows need_abs in both modes
   if (ordered && need_abs)
-    return bwd_go<true, true, 8, BATCH, PERSIST, false>(ctx, "raster_bwd_ordered", pb, bb, T,
-                                                        width, height, bg, final_t, n_contrib,
-                                                        dimage, slots, bd, counter, pc);
+    return bwd_ordered_go<true, BATCH, PERSIST>(ctx, pb, bb, T, width, height, bg, final_t,
+                                                n_contrib, dimage, slots, bd, counter, pc);
   if (ordered)
-    return bwd_go<true, false, 8, BATCH, PERSIST, false>(ctx, "raster_bwd_ordered", pb, bb, T,
-                                                         width, height, bg, final_t, n_contrib,
-                                                         dimage, slots, bd, counter, pc);
+    return bwd_ordered_go<false, BATCH, PERSIST>(ctx, pb, bb, T, width, height, bg, final_t,
+                                                 n_contrib, dimage, slots, bd, counter, pc);
   if (rv.rows)
     return bwd_rows_pick<BATCH, PERSIST, true>(ctx, rv, pb, bb, T, width, height, bg, final_t,
                                                n_contrib, dimage, slots, need_abs, bd, counter);
@@ -914,7 +1054,7 @@ void raster_backward_counted(splat_ctx* ctx, const ProjBuffers& pb, const BinBuf
                              const float* final_t, const uint32_t* n_contrib,
                              const float* dimage, float* slots, unsigned long long* pairs) {
   const unsigned T = bb.tiles_x * bb.tiles_y;
-  launch(ctx, "raster_bwd_count", raster_bwd_kernel<false, false, 32, false, false, true, true>,
+  launch(ctx, "raster_bwd_count", raster_bwd_kernel<false, 32, false, false, true, true>,
          dim3(T), dim3(256), 0, (const float4*)pb.rec, (const uint32_t*)bb.tile_start,
          (const uint32_t*)nullptr, (const uint32_t*)bb.sorted_gauss,
          (const uint32_t*)bb.sorted_entry, T, bb.tiles_x, width, height, bg[0], bg[1], bg[2],
