@@ -18,6 +18,15 @@
 namespace splat {
 namespace {
 
+// Non-persistent launches of one view with few tiles: each wave's own latency bounds them,
+// and registers and LDS are free.  The FEW kernels evaluate a step's pair beside the previous
+// step's state update, without a branch, and take larger batches (fewer barriers).  Forward, in
+// us, FEW with 256-entry batches against 64-entry ones: 256 tiles 39 / 53, 1271 tiles 50 / 57,
+// 4293 tiles 192 / 199, 8160 tiles 185 / 179.  Backward, FEW with 64-entry batches (45 KB of
+// LDS: three workgroups per compute unit) against 32: 256 tiles 97 / 118, 1271 tiles 115 /
+// 140, 4293 tiles 502 / 363; FEW with 32-entry batches lies between at all four sizes.
+constexpr unsigned kFewTilesFwd = 6144;
+constexpr unsigned kFewTilesBwd = 1536;
 constexpr int kOrdBatch = 32;      // entries staged per batch (ordered backward)
 constexpr uint32_t kOrdTerms = 1024;  // pixel terms per slot staged at a time (a tile has 256)
 
@@ -172,6 +181,14 @@ __device__ __forceinline__ bool in_rect(uint32_t rc, uint32_t i, uint32_t j) {
   return ((rc >> i) & (rc >> (16u + j)) & 1u) != 0;
 }
 
+// The record of a Gaussian in registers, on its way to LDS.
+struct StagedRecord {
+  float4 a, b, c;
+};
+__device__ __forceinline__ StagedRecord load_record(const float4* __restrict__ rec, uint32_t g) {
+  return StagedRecord{rec[4 * (size_t)g], rec[4 * (size_t)g + 1], rec[4 * (size_t)g + 2]};
+}
+
 // A row's entry list in LDS holds words {pixel mask of the row's sub-block << 16 | 16 k} for
 // batch entry k: the low half is the entry's byte offset in a float4 array.  Zero is no
 // entry (an entry in a list has a pixel).
@@ -198,6 +215,27 @@ __device__ __forceinline__ void flush_counts(unsigned long long* pairs, int firs
       if (c[q]) atomicAdd(&pairs[first + q], (unsigned long long)c[q]);
 }
 
+// One step of the forward walk for one pixel: evaluate() of src/rasterize.rs:231-244 as far as
+// the alpha test.
+struct FwdPair {
+  uint32_t k16;  // byte offset of the entry
+  bool in;       // the pixel is in the entry's rectangle and 0 <= sigma <= sigma_max
+  float sigma, o, og;
+  __device__ __forceinline__ void evaluate(uint32_t word, uint32_t pixel_bit, const float4* s0,
+                                           const float4* s1, float px, float py) {
+    k16 = word & 0xffffu;
+    const float4 a = at_bytes(s0, k16), b = at_bytes(s1, k16);
+    const float dx = px - a.x;
+    const float dy = py - a.y;
+    sigma = (a.z * dx * dx + b.x * dy * dy) + a.w * dx * dy;  // halved A, C
+    in = ((word & pixel_bit) != 0) & !((sigma < 0.0f) | (sigma > b.z));
+    o = b.y;
+  }
+  __device__ __forceinline__ void exponent(const uint64_t* tab) {
+    og = o * expf_walk_tab(-sigma, tab);  // used where 0 <= sigma <= sigma_max
+  }
+};
+
 // The forward pass is bound by VALU issue, so it is built for few walk steps and few
 // instructions in each: the four 16-lane rows of a wave walk lists of their own (against one
 // walk of the entries that reach the wave's 8x8 block: about a fifth fewer steps), and a list
@@ -206,8 +244,8 @@ __device__ __forceinline__ void flush_counts(unsigned long long* pairs, int firs
 // 256x256: 82 -> 63 us.
 // B: entries per LDS batch; BATCH: tiles of many views (BatchDev); PERSIST: a fixed grid
 // that takes tiles from `counter` until `num_tiles` are done; COUNT: also count pairs
-// into `pairs` (PairCounter).
-template <int B, bool BATCH, bool PERSIST, bool COUNT = false>
+// into `pairs` (PairCounter); FEW: for launches with few tiles (kFewTilesFwd).
+template <int B, bool BATCH, bool PERSIST, bool COUNT = false, bool FEW = false>
 __global__ void __launch_bounds__(256) raster_fwd_kernel(
     const float4* __restrict__ rec, const uint32_t* __restrict__ tile_start,
     const uint32_t* __restrict__ order,
@@ -220,9 +258,10 @@ __global__ void __launch_bounds__(256) raster_fwd_kernel(
   __shared__ uint64_t tab[32];
   __shared__ float4 s0[B], s1[B], s2[B];
   __shared__ uint32_t srect[B];
-  __shared__ uint32_t slist[16][kList];  // per (wave, row): its entries, front to back
+  __shared__ uint32_t slist[16][kList + 1];  // per (wave, row): its entries, front to back
   __shared__ uint32_t s_tile;
   if (threadIdx.x < 32) tab[threadIdx.x] = kExp2Table[threadIdx.x];
+  if (FEW && threadIdx.x < 16) slist[threadIdx.x][kList] = 0u;
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane >> 4;
   const uint32_t pixel_bit = 0x10000u << (lane & 15u);
   const uint32_t* my_list = slist[wave * 4 + row];
@@ -241,18 +280,28 @@ __global__ void __launch_bounds__(256) raster_fwd_kernel(
   bool done = !valid;
   uint32_t pcount[5] = {0, 0, 0, 0, 0};
   const uint32_t start = tile_start[tile], end = tile_start[tile + 1];
+  // The records of a batch are loaded while the batch before it is walked, their Gaussians one
+  // batch earlier still (lanes past the end repeat its last entry).
+  StagedRecord sr{};
+  uint32_t next_g = 0;
+  if (threadIdx.x < B && start < end) {
+    sr = load_record(rec, sorted_gauss[min(start + threadIdx.x, end - 1)]);
+    next_g = sorted_gauss[min(start + B + threadIdx.x, end - 1)];
+  }
   for (uint32_t b0 = start; b0 < end; b0 += B) {
     if (__syncthreads_and(done ? 1 : 0)) break;
     const uint32_t cnt = min((uint32_t)B, end - b0);
-    if (threadIdx.x < cnt) {
-      const uint32_t g = sorted_gauss[b0 + threadIdx.x];
-      const float4 a = rec[4 * g], b = rec[4 * g + 1], c = rec[4 * g + 2];
-      s0[threadIdx.x] = half_conic0(a);
-      s1[threadIdx.x] = half_conic1(b);
-      s2[threadIdx.x] = c;
-      srect[threadIdx.x] = entry_rect(a, b, c, ti);
+    if (threadIdx.x < B) {
+      s0[threadIdx.x] = half_conic0(sr.a);
+      s1[threadIdx.x] = half_conic1(sr.b);
+      s2[threadIdx.x] = sr.c;
+      srect[threadIdx.x] = entry_rect(sr.a, sr.b, sr.c, ti);
     }
     __syncthreads();
+    if (threadIdx.x < B && b0 + B < end) {
+      sr = load_record(rec, next_g);
+      next_g = sorted_gauss[min(b0 + 2 * B + threadIdx.x, end - 1)];
+    }
     // Predicated form of the per-pixel walk (src/rasterize.rs:262-290): every decision of
     // evaluate() and the T_MIN test is a lane predicate; only the exp is skipped when no
     // lane of the wave needs it.  The four rows of a wave walk, side by side and each in
@@ -278,28 +327,9 @@ __global__ void __launch_bounds__(256) raster_fwd_kernel(
       }
       __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
       uint32_t last = 0xffffffffu;  // byte offset of the last composited entry of this list
-      for (uint32_t t = 0; t < steps; t++) {
-        const uint32_t le = my_list[t], k16 = le & 0xffffu;
-        const float4 a = at_bytes(s0, k16), b = at_bytes(s1, k16);
-        const float dx = px - a.x;
-        const float dy = py - a.y;
-        const float sigma = (a.z * dx * dx + b.x * dy * dy) + a.w * dx * dy;  // halved A, C
-        const bool pass1 =
-            (!done) & ((le & pixel_bit) != 0) & !((sigma < 0.0f) | (sigma > b.z));
-        if (COUNT) {
-          const uint64_t b1 = __ballot(pass1);
-          pcount[0]++;
-          if (!b1) continue;
-          pcount[1]++;
-          pcount[2] += (uint32_t)__popcll(b1);
-        } else if (__builtin_amdgcn_ballot_w64(pass1) == 0) {
-          continue;
-        }
-        const float4 c = at_bytes(s2, k16);
-        const float G = expf_walk_tab(-sigma, tab);  // used where 0 <= sigma <= sigma_max
-        const float og = b.y * G;
-        const bool pass2 = pass1 & !(og < kAlphaMin);
-        const float alpha = rmin(og, kAlphaMax);
+      const auto blend = [&](const FwdPair& p, bool pass1, float4 c) {
+        const bool pass2 = pass1 & !(p.og < kAlphaMin);
+        const float alpha = rmin(p.og, kAlphaMax);
         const float test_t = T * (1.0f - alpha);
         const bool stop = test_t < kTMin;
         done = done | (pass2 & stop);
@@ -313,7 +343,40 @@ __global__ void __launch_bounds__(256) raster_fwd_kernel(
         c1 = comp ? c1 + w * c.z : c1;
         c2 = comp ? c2 + w * c.w : c2;
         T = comp ? test_t : T;
-        last = comp ? k16 : last;
+        last = comp ? p.k16 : last;
+      };
+      if (FEW) {
+        // the pair of the next step is evaluated beside the blend of this one
+        FwdPair p;
+        p.evaluate(my_list[0], pixel_bit, s0, s1, px, py);
+        p.exponent(tab);
+        uint32_t next = my_list[1];
+        for (uint32_t t = 0; t < steps; t++) {
+          const FwdPair now = p;
+          const float4 c = at_bytes(s2, now.k16);
+          p.evaluate(next, pixel_bit, s0, s1, px, py);
+          p.exponent(tab);
+          next = my_list[min(t + 2, (uint32_t)kList)];
+          blend(now, !done & now.in, c);
+        }
+      } else {
+        for (uint32_t t = 0; t < steps; t++) {
+          FwdPair p;
+          p.evaluate(my_list[t], pixel_bit, s0, s1, px, py);
+          const bool pass1 = !done & p.in;
+          if (COUNT) {
+            const uint64_t b1 = __ballot(pass1);
+            pcount[0]++;
+            if (!b1) continue;
+            pcount[1]++;
+            pcount[2] += (uint32_t)__popcll(b1);
+          } else if (__builtin_amdgcn_ballot_w64(pass1) == 0) {
+            continue;
+          }
+          const float4 c = at_bytes(s2, p.k16);
+          p.exponent(tab);
+          blend(p, pass1, c);
+        }
       }
       if (last != 0xffffffffu) nc = b0 - start + (last >> 4) + 1;
     }
@@ -481,67 +544,66 @@ __device__ __forceinline__ float row_sums9(float v0, float v1, float v2, float v
 // The pixel state uses acc0..2 for A; lc and last_alpha are unused.  Returns the row sums of
 // the slot terms as row_sums9 leaves them in the lanes (with ABS, slots 9 and 10 in the rows'
 // lanes 13 and 11).
-// COUNT: cnt[0..3] += visit, active visit, evaluated and passing pairs.
-template <bool ABS, bool COUNT = false>
-__device__ __forceinline__ float pair_sums_fast(PixBack& s, bool act, float4 r0, float4 r1,
-                                                const float4* r2at, float px, float py,
-                                                const uint64_t* tab, bool bg,
-                                                uint32_t* cnt = nullptr) {
-  const float dx = px - r0.x;
-  const float dy = py - r0.y;
-  const float sigma = (r0.z * dx * dx + r1.x * dy * dy) + r0.w * dx * dy;  // halved A, C
-  const bool p1 = act & !((sigma < 0.0f) | (sigma > r1.z));
-  if (COUNT) {
-    const uint64_t b1 = __ballot(p1);
-    cnt[0]++;
-    if (!b1) return 0.0f;
-    cnt[1]++;
-    cnt[2] += (uint32_t)__popcll(b1);
-  } else if (__builtin_amdgcn_ballot_w64(p1) == 0) {
-    return 0.0f;
+// The step in two parts: evaluate() and exponent() depend on the pair alone, sums() on the
+// pixel's state.
+template <bool ABS>
+struct BwdPair {
+  bool in;  // the pixel is a candidate of the entry and 0 <= sigma <= sigma_max
+  float dx, dy, sigma, o, G;
+  __device__ __forceinline__ void evaluate(bool act, float4 r0, float4 r1, float px, float py) {
+    dx = px - r0.x;
+    dy = py - r0.y;
+    sigma = (r0.z * dx * dx + r1.x * dy * dy) + r0.w * dx * dy;  // halved A, C
+    in = act & !((sigma < 0.0f) | (sigma > r1.z));
+    o = r1.y;
   }
-  const float4 r2 = *r2at;
-  const float G = expf_walk_tab(-sigma, tab);  // used where 0 <= sigma <= sigma_max
-  const float o = r1.y;
-  const float og = o * G;
-  const bool p2 = p1 & !(og < kAlphaMin);
-  const bool p3 = p2 & (og < kAlphaMax);
-  if (COUNT) cnt[3] += (uint32_t)__popcll(__ballot(p2));
-  const float alpha = rmin(og, kAlphaMax);
-  const float den = 1.0f - alpha;
-  const float inv = __builtin_amdgcn_rcpf(den);
-  const float q0 = s.t * inv;
-  const float t = fmaf(fmaf(-q0, den, s.t), inv, q0);
-  const float e0 = r2.y - s.acc0, e1 = r2.z - s.acc1, e2 = r2.w - s.acc2;
-  float dalpha = e0 * s.d0;
-  dalpha = fmaf(e1, s.d1, dalpha);
-  dalpha = fmaf(e2, s.d2, dalpha);
-  if (bg) {  // uniform: a kernel argument
-    const float f0 = s.t_final * inv;
-    const float tf = fmaf(fmaf(-f0, den, s.t_final), inv, f0);
-    dalpha = fmaf(dalpha, t, -tf * s.bg_dot);
-  } else {
-    dalpha *= t;
+  __device__ __forceinline__ void exponent(const uint64_t* tab) {
+    G = expf_walk_tab(-sigma, tab);  // used where 0 <= sigma <= sigma_max
   }
-  const float q = p3 ? -(o * dalpha) * G : 0.0f;
-  const float w = p2 ? alpha * t : 0.0f;
-  s.t = p2 ? t : s.t;
-  s.acc0 = p2 ? fmaf(alpha, e0, s.acc0) : s.acc0;
-  s.acc1 = p2 ? fmaf(alpha, e1, s.acc1) : s.acc1;
-  s.acc2 = p2 ? fmaf(alpha, e2, s.acc2) : s.acc2;
-  const float qdx = q * dx, qdy = q * dy;
-  constexpr uint64_t kUpper = 0xccccccccccccccccull, kLast = 0x8000800080008000ull;
-  float out = row_sums9(qdx, qdy, qdx * dx, qdx * dy, qdy * dy, p3 ? G * dalpha : 0.0f, w * s.d0,
-                        w * s.d1, w * s.d2, kUpper, kLast);
-  if (ABS) {
-    const float e9 = row_allsum16(fabsf(fmaf(2.0f * r0.z, qdx, r0.w * qdy)));
-    const float e10 = row_allsum16(fabsf(fmaf(r0.w, qdx, (2.0f * r1.x) * qdy)));
-    const uint32_t l16 = threadIdx.x & 15u;
-    out = l16 == 13 ? e9 : out;
-    out = l16 == 11 ? e10 : out;
+  // r0z, r0w, r1x: the (halved) conic, read with ABS only.  passing (COUNT): += passing pairs.
+  template <bool COUNT>
+  __device__ __forceinline__ float sums(PixBack& s, float4 r2, bool bg, float r0z, float r0w,
+                                        float r1x, uint32_t* passing) const {
+    const float og = o * G;
+    const bool p2 = in & !(og < kAlphaMin);
+    const bool p3 = p2 & (og < kAlphaMax);
+    if (COUNT) *passing += (uint32_t)__popcll(__ballot(p2));
+    const float alpha = rmin(og, kAlphaMax);
+    const float den = 1.0f - alpha;
+    const float inv = __builtin_amdgcn_rcpf(den);
+    const float q0 = s.t * inv;
+    const float t = fmaf(fmaf(-q0, den, s.t), inv, q0);
+    const float e0 = r2.y - s.acc0, e1 = r2.z - s.acc1, e2 = r2.w - s.acc2;
+    float dalpha = e0 * s.d0;
+    dalpha = fmaf(e1, s.d1, dalpha);
+    dalpha = fmaf(e2, s.d2, dalpha);
+    if (bg) {  // uniform: a kernel argument
+      const float f0 = s.t_final * inv;
+      const float tf = fmaf(fmaf(-f0, den, s.t_final), inv, f0);
+      dalpha = fmaf(dalpha, t, -tf * s.bg_dot);
+    } else {
+      dalpha *= t;
+    }
+    const float q = p3 ? -(o * dalpha) * G : 0.0f;
+    const float w = p2 ? alpha * t : 0.0f;
+    s.t = p2 ? t : s.t;
+    s.acc0 = p2 ? fmaf(alpha, e0, s.acc0) : s.acc0;
+    s.acc1 = p2 ? fmaf(alpha, e1, s.acc1) : s.acc1;
+    s.acc2 = p2 ? fmaf(alpha, e2, s.acc2) : s.acc2;
+    const float qdx = q * dx, qdy = q * dy;
+    constexpr uint64_t kUpper = 0xccccccccccccccccull, kLast = 0x8000800080008000ull;
+    float out = row_sums9(qdx, qdy, qdx * dx, qdx * dy, qdy * dy, p3 ? G * dalpha : 0.0f,
+                          w * s.d0, w * s.d1, w * s.d2, kUpper, kLast);
+    if (ABS) {
+      const float e9 = row_allsum16(fabsf(fmaf(2.0f * r0z, qdx, r0w * qdy)));
+      const float e10 = row_allsum16(fabsf(fmaf(r0w, qdx, (2.0f * r1x) * qdy)));
+      const uint32_t l16 = threadIdx.x & 15u;
+      out = l16 == 13 ? e9 : out;
+      out = l16 == 11 ? e10 : out;
+    }
+    return out;
   }
-  return out;
-}
+};
 
 // A pixel's state at the start of the backward walk.  valid: inside the image.
 __device__ __forceinline__ PixBack pixel_back(const TileGeom& tg, uint32_t i, uint32_t j,
@@ -581,7 +643,9 @@ __device__ __forceinline__ PixBack pixel_back(const TileGeom& tg, uint32_t i, ui
 // 16-lane row walks its own entry list; otherwise the wave walks the entries that reach any
 // of its rows (the same sums either way).  COUNT: also count pairs into `pairs`
 // (PairCounter).
-template <bool ABS, int B, bool BATCH, bool PERSIST, bool ROWS, bool COUNT = false>
+// FEW: for launches with few tiles (kFewTilesBwd); rows only.
+template <bool ABS, int B, bool BATCH, bool PERSIST, bool ROWS, bool COUNT = false,
+          bool FEW = false>
 __global__ void __launch_bounds__(256) raster_bwd_kernel(
     const float4* __restrict__ rec, const uint32_t* __restrict__ tile_start,
     const uint32_t* __restrict__ order,
@@ -590,14 +654,14 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
     float bg2, const float* __restrict__ final_t, const uint32_t* __restrict__ n_contrib,
     const float* __restrict__ dimage, float* __restrict__ slots, BatchDev bd,
     uint32_t* __restrict__ counter, unsigned long long* __restrict__ pairs) {
-  static_assert(B <= 32, "a list is built by half a wave");
+  static_assert(B <= 32 || (B == 64 && ROWS), "a list is built by half a wave, or by a wave");
   // words per entry in `slots` and per row partial: the absolute sums (9, 10) only when asked
   constexpr uint32_t SS = ABS ? kSlots : 9;
   __shared__ uint64_t tab[32];
   __shared__ float4 s0[B], s1[B], s2[B];
-  __shared__ uint32_t srect[B];
+  __shared__ uint32_t srect[B], sentry[B];
   __shared__ __align__(4) uint8_t svisit[B][4];  // per entry and wave: the rows that wrote a partial
-  __shared__ uint32_t slist[16][B];    // per (wave, row): its entries, back to front
+  __shared__ uint32_t slist[16][B + 1];  // per (wave, row): its entries, back to front
   __shared__ uint32_t smax_last;
   __shared__ uint32_t s_tile;
   // Partials of the batch, [entry][wave, row][word]; only those named by svisit are written
@@ -606,6 +670,7 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
   // whether the background term (T_final bg . dL) can be non-zero for a finite dL
   const bool bg_any = (bg0 != 0.0f) | (bg1 != 0.0f) | (bg2 != 0.0f);
   if (threadIdx.x < 32) tab[threadIdx.x] = kExp2Table[threadIdx.x];
+  if (FEW && threadIdx.x < 16) slist[threadIdx.x][B] = 0u;
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, row = lane >> 4;
   const uint32_t l16 = lane & 15u;
   const uint32_t pixel_bit = 0x10000u << l16;
@@ -648,45 +713,67 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
     for (int r = 0; r < 4; r++) row_last[r] = (uint32_t)__builtin_amdgcn_readlane((int)m, 16 * r);
   }
   const uint32_t wave_last = max(max(row_last[0], row_last[1]), max(row_last[2], row_last[3]));
-  // Batches walk [0, kmax) from the back.
+  // Batches walk [0, kmax) from the back.  A batch's records are loaded while the batch behind
+  // it is summed, their Gaussians and entry ids while it is walked (lanes past a batch's end
+  // repeat its last entry).
+  StagedRecord sr{};
+  uint32_t next_g = 0, entry_id = 0, next_id = 0;
+  const auto batch_index = [&](int32_t h) {  // of the batch that ends at h
+    const int32_t l = max(h - B, 0);
+    return start + (uint32_t)min(l + (int32_t)threadIdx.x, h - 1);
+  };
+  if (threadIdx.x < B && kmax > 0) {
+    const uint32_t at = batch_index((int32_t)kmax);
+    next_g = sorted_gauss[at];
+    entry_id = sorted_entry[at];
+    sr = load_record(rec, next_g);
+  }
   for (int32_t hi = (int32_t)kmax; hi > 0; hi -= B) {
     const int32_t lo = max(hi - B, 0);
     const uint32_t cnt = (uint32_t)(hi - lo);
     __syncthreads();
-    if (threadIdx.x < cnt) {
-      const uint32_t g = sorted_gauss[start + lo + threadIdx.x];
-      const float4 a = rec[4 * g], b = rec[4 * g + 1], c = rec[4 * g + 2];
-      s0[threadIdx.x] = half_conic0(a);
-      s1[threadIdx.x] = half_conic1(b);
-      s2[threadIdx.x] = c;
-      srect[threadIdx.x] = entry_rect(a, b, c, ti);
+    if (threadIdx.x < B) {
+      s0[threadIdx.x] = half_conic0(sr.a);
+      s1[threadIdx.x] = half_conic1(sr.b);
+      s2[threadIdx.x] = sr.c;
+      srect[threadIdx.x] = entry_rect(sr.a, sr.b, sr.c, ti);
+      sentry[threadIdx.x] = entry_id;
+      if (lo > 0) {
+        const uint32_t at = batch_index(lo);
+        next_g = sorted_gauss[at];
+        next_id = sorted_entry[at];
+      }
     }
     __syncthreads();
     // Each 16-lane row walks, back to front, only the batch entries that reach its 4x4
     // sub-block and precede the row's last contributor; the four rows of a wave walk
-    // their own lists side by side.  Lanes 0-31 build the lists of rows 0 and 1, lanes
-    // 32-63 those of rows 2 and 3, one entry per lane.
-    const uint32_t kl = lane & 31u, half = lane >> 5;
+    // their own lists side by side.  One entry per lane; with batches of up to 32, lanes 0-31
+    // build the lists of rows 0 and 1, lanes 32-63 those of rows 2 and 3.
+    constexpr uint32_t kHalf = B <= 32 ? 32 : 64;
+    const uint32_t kl = lane % kHalf, half = lane / kHalf;
     const uint32_t rc = kl < cnt ? srect[min(kl, (uint32_t)B - 1u)] : 0u;
     uint32_t steps = 0, visit = 0;
     uint64_t wave_todo = 0;  // !ROWS: the wave's entries, walked from the top bit down
     if (ROWS) {
 #pragma unroll
-      for (uint32_t r = 0; r < 2; r++) {
-        const uint32_t last = half ? row_last[r + 2] : row_last[r];
-        const uint32_t pm = lo + kl < last ? row_mask(rc, wave, half * 2 + r) : 0u;
+      for (uint32_t r = 0; r < kHalf / 16; r++) {
+        const uint32_t q = half * 2 + r;  // the row
+        const uint32_t last = half ? row_last[(r + 2) % 4] : row_last[r];
+        const uint32_t pm = lo + kl < last ? row_mask(rc, wave, q) : 0u;
         const uint64_t m2 = __ballot(pm != 0);
-        const uint32_t lo_half = (uint32_t)m2, hi_half = (uint32_t)(m2 >> 32);
-        const uint32_t m = half ? hi_half : lo_half;
-        const uint32_t len = (uint32_t)__popc(m);
-        uint32_t* list = slist[wave * 4 + half * 2 + r];
+        uint64_t m = m2;
+        if (kHalf == 32) m = half ? m2 >> 32 : m2 & 0xffffffffull;
+        const uint32_t len = (uint32_t)__popcll(m);
+        uint32_t* list = slist[wave * 4 + q];
         // entry kl sits behind the later entries of the batch
-        if (pm) list[__popc(m >> kl) - 1] = (pm << 16) | (kl << 4);
+        if (pm) list[__popcll(m >> kl) - 1] = (pm << 16) | (kl << 4);
         if (kl >= len && kl < (uint32_t)B) list[kl] = 0u;  // past the end: no entry
         if (pm) visit |= 1u << r;
-        steps = max(steps, max((uint32_t)__popc(lo_half), (uint32_t)__popc(hi_half)));
+        steps = max(steps, kHalf == 32 ? max((uint32_t)__popc((uint32_t)m2),
+                                             (uint32_t)__popc((uint32_t)(m2 >> 32)))
+                                       : len);
       }
-      visit |= (uint32_t)__shfl((int)visit, (int)(kl + 32), 64) << 2;  // for lanes 0-31
+      if (kHalf == 32) visit |= (uint32_t)__shfl((int)visit, (int)(kl + 32), 64) << 2;
     } else {
       const bool on = lane < cnt && lo + lane < wave_last && wave_touches(rc, wave);
       wave_todo = __ballot(on);
@@ -698,26 +785,74 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     const uint32_t* my_list = slist[wave * 4 + row];
     const uint32_t last16 = s.last > (uint32_t)lo ? min(s.last - lo, (uint32_t)B) << 4 : 0u;
-    for (uint32_t t = 0; t < steps; t++) {
-      uint32_t k16;
-      bool has = true, act;
-      if (ROWS) {
-        const uint32_t le = my_list[t];
-        k16 = le & 0xffffu;
-        has = le != 0;
-        act = ((le & pixel_bit) != 0) & (k16 < last16);
-      } else {
-        const uint32_t kk = 63u - (uint32_t)__builtin_clzll(wave_todo);
-        wave_todo &= ~(1ull << kk);
-        k16 = kk << 4;
-        act = (k16 < last16) & in_rect(srect[kk], i, j);
+    const uint32_t my_red = (wave * 4 + row) * SS + wslot;
+    if (FEW) {
+      // the pair of the next step is evaluated beside the sums of this one
+      uint32_t le = my_list[0], next = my_list[1];
+      BwdPair<ABS> p;
+      const auto prepare = [&] {
+        const uint32_t k16 = le & 0xffffu;
+        p.evaluate(((le & pixel_bit) != 0) & (k16 < last16), at_bytes(s0, k16), at_bytes(s1, k16),
+                   px, py);
+        p.exponent(tab);
+      };
+      prepare();
+      for (uint32_t t = 0; t < steps; t++) {
+        const BwdPair<ABS> now = p;
+        const uint32_t k16 = le & 0xffffu;
+        const bool has = le != 0;
+        const float4 r2 = at_bytes(s2, k16);
+        float r0z = 0, r0w = 0, r1x = 0;
+        if (ABS) {
+          const float4 r0 = at_bytes(s0, k16);
+          r0z = r0.z;
+          r0w = r0.w;
+          r1x = at_bytes(s1, k16).x;
+        }
+        le = next;
+        next = my_list[min(t + 2, (uint32_t)B)];
+        prepare();
+        const float out = now.template sums<false>(s, r2, bg_any, r0z, r0w, r1x, nullptr);
+        if (has & writer) red[k16 * SS + my_red] = out;
       }
-      const float4* r2at = reinterpret_cast<const float4*>(reinterpret_cast<const char*>(s2) + k16);
-      const float out = pair_sums_fast<ABS, COUNT>(s, act, at_bytes(s0, k16), at_bytes(s1, k16),
-                                                   r2at, px, py, tab, bg_any, pcount);
-      if (has & writer) red[k16 * SS + (wave * 4 + row) * SS + wslot] = out;
+    } else {
+      for (uint32_t t = 0; t < steps; t++) {
+        uint32_t k16;
+        bool has = true, act;
+        if (ROWS) {
+          const uint32_t le = my_list[t];
+          k16 = le & 0xffffu;
+          has = le != 0;
+          act = ((le & pixel_bit) != 0) & (k16 < last16);
+        } else {
+          const uint32_t kk = 63u - (uint32_t)__builtin_clzll(wave_todo);
+          wave_todo &= ~(1ull << kk);
+          k16 = kk << 4;
+          act = (k16 < last16) & in_rect(srect[kk], i, j);
+        }
+        BwdPair<ABS> p;
+        const float4 r0 = at_bytes(s0, k16), r1 = at_bytes(s1, k16);
+        p.evaluate(act, r0, r1, px, py);
+        float out = 0.0f;
+        const uint64_t b1 = __builtin_amdgcn_ballot_w64(p.in);
+        if (COUNT) pcount[0]++;
+        if (b1) {
+          if (COUNT) {
+            pcount[1]++;
+            pcount[2] += (uint32_t)__popcll(b1);
+          }
+          const float4 r2 = at_bytes(s2, k16);
+          p.exponent(tab);
+          out = p.template sums<COUNT>(s, r2, bg_any, r0.z, r0.w, r1.x, &pcount[3]);
+        }
+        if (has & writer) red[k16 * SS + my_red] = out;
+      }
     }
     __syncthreads();
+    entry_id = next_id;
+    // assigned on every path: the registers are free during the walk
+    sr = StagedRecord{};
+    if (threadIdx.x < B) sr = load_record(rec, next_g);
     // Sum the batch's partials and write its slots: 16 lanes per entry, lane = slot.
     const uint32_t slot = threadIdx.x & 15u;
     for (uint32_t e0 = 0; e0 < cnt; e0 += 16) {
@@ -733,7 +868,7 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
           acc += p[(uint32_t)__builtin_ctz(rows) * SS];
           rows &= rows - 1;
         }
-        // pair_sums_fast's products: slots 0, 1 combine both position sums with the conic
+        // the products' sums: slots 0, 1 combine both position sums with the conic
         const float other = dpp_row<0xb1>(acc);  // lane ^ 1
         if (slot == 0)
           acc = -fmaf(2.0f * a.z, acc, a.w * other);
@@ -741,7 +876,7 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
           acc = -fmaf(a.w, other, (2.0f * b.x) * acc);
         else if (slot == 2 || slot == 4)
           acc *= 0.5f;
-        slots[(size_t)sorted_entry[start + lo + kk] * SS + slot] = acc;
+        slots[(size_t)sentry[kk] * SS + slot] = acc;
       }
     }
   }
@@ -936,6 +1071,14 @@ template <int B, bool BATCH, bool PERSIST>
 void fwd_go(splat_ctx* ctx, const ProjBuffers& pb, const BinBuffers& bb, unsigned T,
             uint32_t width, uint32_t height, const float bg[3], float* image, float* final_t,
             uint32_t* n_contrib, const BatchDev& bd, uint32_t* counter, unsigned per_cu) {
+  if constexpr (!BATCH && !PERSIST) {
+    if (T <= kFewTilesFwd)
+      return launch(ctx, "raster_fwd", raster_fwd_kernel<256, false, false, false, true>, dim3(T),
+                    dim3(256), 0, (const float4*)pb.rec, (const uint32_t*)bb.tile_start,
+                    (const uint32_t*)bb.tile_order, (const uint32_t*)bb.sorted_gauss, T,
+                    bb.tiles_x, width, height, bg[0], bg[1], bg[2], image, final_t, n_contrib, bd,
+                    counter, (unsigned long long*)nullptr);
+  }
   if (PERSIST) fill_u32(ctx, counter, kXcds, 0u);
   const unsigned grid = PERSIST ? persistent_grid(ctx, per_cu, T) : T;
   launch(ctx, "raster_fwd", raster_fwd_kernel<B, BATCH, PERSIST>, dim3(grid), dim3(256), 0,
@@ -949,6 +1092,16 @@ void bwd_go(splat_ctx* ctx, const ProjBuffers& pb, const BinBuffers& bb, unsigne
             uint32_t width, uint32_t height, const float bg[3], const float* final_t,
             const uint32_t* n_contrib, const float* dimage, float* slots, const BatchDev& bd,
             uint32_t* counter, unsigned per_cu) {
+  if constexpr (!BATCH && !PERSIST) {
+    if (T <= kFewTilesBwd)
+      return launch(ctx, "raster_bwd",
+                    raster_bwd_kernel<ABS, 64, false, false, true, false, true>, dim3(T), dim3(256),
+                    0, (const float4*)pb.rec, (const uint32_t*)bb.tile_start,
+                    (const uint32_t*)bb.tile_order, (const uint32_t*)bb.sorted_gauss,
+                    (const uint32_t*)bb.sorted_entry, T, bb.tiles_x, width, height, bg[0], bg[1],
+                    bg[2], final_t, n_contrib, dimage, slots, bd, counter,
+                    (unsigned long long*)nullptr);
+  }
   if (PERSIST) fill_u32(ctx, counter, kXcds, 0u);
   const unsigned grid = PERSIST ? persistent_grid(ctx, per_cu, T) : T;
   launch(ctx, "raster_bwd", raster_bwd_kernel<ABS, BF, BATCH, PERSIST, ROWS>, dim3(grid),
