@@ -88,7 +88,7 @@ struct splat_batch {
   std::vector<uint32_t> plan_views;
   BatchDev bd{};
   size_t work = 0, tiles = 0, pixels = 0;
-  unsigned loss_blocks_total = 0;
+  unsigned loss_blocks_total = 0, loss_rows = 0;
   // captured step
   BatchKey key;
   hipGraphExec_t exec = nullptr;
@@ -119,7 +119,6 @@ void build_plan(splat_batch* b, const std::vector<uint32_t>& views) {
     work_base[k] = (uint32_t)work;
     tile_base[k] = (uint32_t)tiles;
     pix_base[k] = (uint32_t)pix;
-    lbb[k] = (uint32_t)lblocks;
     tiles_x[k] = (W + kTile - 1) / kTile;
     SPLAT_REQUIRE((size_t)tiles_x[k] * ((H + kTile - 1) / kTile) < kMaxViewTiles,
                   "view too large for radix binning");
@@ -130,7 +129,11 @@ void build_plan(splat_batch* b, const std::vector<uint32_t>& views) {
     work += b->scenes[v.scene].n;
     tiles += (size_t)tiles_x[k] * ((H + kTile - 1) / kTile);
     pix += (size_t)W * H;
-    lblocks += loss_blocks(W, H);
+  }
+  const unsigned lrows = loss_rows(width.data(), height.data(), P);
+  for (uint32_t k = 0; k < P; k++) {
+    lbb[k] = (uint32_t)lblocks;
+    lblocks += loss_blocks(width[k], height[k], lrows);
   }
   SPLAT_REQUIRE(work < 0xffffffffull && pix < 0xffffffffull / 3 && tiles < 0xffffffffull,
                 "batch too large");
@@ -191,6 +194,7 @@ void build_plan(splat_batch* b, const std::vector<uint32_t>& views) {
   b->tiles = tiles;
   b->pixels = pix;
   b->loss_blocks_total = (unsigned)lblocks;
+  b->loss_rows = lrows;
 }
 
 struct BatchBufs {
@@ -262,7 +266,7 @@ void enqueue(splat_batch* b, const BatchBufs& x, const splat_batch_step_params& 
                          x.scan_sums, x.status, &bd);
   raster_forward(ctx, x.pb, x.bb, 0, 0, p.background, x.image, x.final_t, x.n_contrib, fwd, &bd,
                  x.counter);
-  loss_forward_backward_batch(ctx, x.image, bd, b->loss_blocks_total, b->pixels * 3,
+  loss_forward_backward_batch(ctx, x.image, bd, b->loss_blocks_total, b->loss_rows, b->pixels * 3,
                               p.lambda_dssim, x.dimage, x.scratch, x.losses);
   raster_backward(ctx, x.pb, x.bb, 0, 0, p.background, x.final_t, x.n_contrib, x.dimage,
                   p.ordered_backward != 0, x.slots, false, bwd, &bd, x.counter);
@@ -504,7 +508,7 @@ int splat_batch_tune(splat_batch* b, const uint32_t* views, uint32_t nviews,
     RasterVariant def;
     raster_forward(ctx, x.pb, x.bb, 0, 0, p->background, x.image, x.final_t, x.n_contrib, def,
                    &b->bd, x.counter);
-    loss_forward_backward_batch(ctx, x.image, b->bd, b->loss_blocks_total, b->pixels * 3,
+    loss_forward_backward_batch(ctx, x.image, b->bd, b->loss_blocks_total, b->loss_rows, b->pixels * 3,
                                 p->lambda_dssim, x.dimage, x.scratch, nullptr);
     const RasterTune tr = tune_raster(ctx, x.pb, x.bb, 0, 0, p->background, x.image, x.final_t,
                                       x.n_contrib, x.dimage, p->ordered_backward != 0, x.slots,

@@ -605,14 +605,16 @@ hipError_t loss_launch_bare(hipStream_t stream, const float* pred, const float* 
                             float* loss_out, float* scratch);
 // Resolves this device's address of the no-allocation scratch array (once per device).
 int noalloc_setup(int device);
-// Blocks of the loss kernels for one image (the batched grid is the sum over pairs).
-unsigned loss_blocks(uint32_t width, uint32_t height);
+// Rows per workgroup of the loss kernels for a launch over the given images, and the
+// workgroups of one image (the batched grid is the sum over pairs).
+unsigned loss_rows(const uint32_t* width, const uint32_t* height, size_t images);
+unsigned loss_blocks(uint32_t width, uint32_t height, unsigned rows);
 // Batched: loss and dL/dimage of every pair in two launches; scratch holds 3 maps of
 // total_values floats (pixels x 3 over all pairs) and 2 floats per block; losses (optional,
 // device) gets one value per pair.
 void loss_forward_backward_batch(splat_ctx* ctx, const float* pred, const BatchDev& bd,
-                                 unsigned total_blocks, size_t total_values, float lambda,
-                                 float* dimage, float* scratch, float* losses);
+                                 unsigned total_blocks, unsigned rows, size_t total_values,
+                                 float lambda, float* dimage, float* scratch, float* losses);
 // The loss value of the last loss_forward_backward on `scratch`, into device memory
 // (`out_dev`, or dyn->loss_out when `dyn` is given).
 void loss_value_to(splat_ctx* ctx, const float* scratch, uint32_t width, uint32_t height,

@@ -20,7 +20,15 @@ namespace {
 
 constexpr int kStrip = 256;
 constexpr int kHalo = 15;        // 5 pixels x 3 channels
-constexpr int kRowsPerBlock = 32;
+
+// Rows per workgroup.  A workgroup of r rows blurs r + 10 (the halo), one after the other, and
+// three workgroups share a compute unit, so large images want long chunks and small images
+// enough workgroups.  The shortest chunk that keeps a launch to kLossBlocks workgroups was
+// within 5% of the best of 2..64 rows at every size measured (both passes, in us, fixed 32
+// rows before / this rule): 256x256 89 / 30, 400x304 90 / 37, 800x600 97 / 50, 1024x768
+// 103 / 67, 1297x840 104 / 84, 1600x1200 120 / 112, 1920x1080 121 / 122.
+constexpr unsigned kLossBlocks = 950;
+constexpr unsigned kMinLossRows = 2, kMaxLossRows = 64;
 
 struct Taps {
   float k[11];
@@ -133,7 +141,7 @@ __global__ void __launch_bounds__(256) ssim_stats_kernel(const float* __restrict
                                                          float* __restrict__ d_exy,
                                                          float2* __restrict__ partial,
                                                          const StepDyn* __restrict__ dyn,
-                                                         BatchDev bd) {
+                                                         BatchDev bd, int rows) {
   if (dyn) yin = dyn->target;
   size_t pix0;
   uint32_t pair;
@@ -153,8 +161,8 @@ __global__ void __launch_bounds__(256) ssim_stats_kernel(const float* __restrict
   const int q0 = lb.bx * kStrip;
   const int q = q0 + threadIdx.x;
   const bool col_ok = q < width3;
-  const int ybeg = lb.by * kRowsPerBlock;
-  const int yend = min(ybeg + kRowsPerBlock, (int)H);
+  const int ybeg = lb.by * rows;
+  const int yend = min(ybeg + rows, (int)H);
   float h[5][11];
 #pragma unroll
   for (int m = 0; m < 5; m++)
@@ -318,7 +326,7 @@ __global__ void __launch_bounds__(256) ssim_grad_kernel(const float* __restrict_
                                                         float inv_n, float w1, float lambda,
                                                         float* __restrict__ grad,
                                                         const StepDyn* __restrict__ dyn,
-                                                        BatchDev bd, StepLossReport rep) {
+                                                        BatchDev bd, StepLossReport rep, int rows) {
   if (dyn) yin = dyn->target;
   // the partial sums of pass 1 are complete: workgroup 0 also writes the step's report
   if (rep.reports && blockIdx.x == 0 && blockIdx.y == 0) write_step_report(rep, lambda, dyn);
@@ -343,8 +351,8 @@ __global__ void __launch_bounds__(256) ssim_grad_kernel(const float* __restrict_
   const int q0 = lb.bx * kStrip;
   const int q = q0 + threadIdx.x;
   const bool col_ok = q < width3;
-  const int ybeg = lb.by * kRowsPerBlock;
-  const int yend = min(ybeg + kRowsPerBlock, (int)H);
+  const int ybeg = lb.by * rows;
+  const int yend = min(ybeg + rows, (int)H);
   float h[3][11];
 #pragma unroll
   for (int m = 0; m < 3; m++)
@@ -482,13 +490,30 @@ __global__ void __launch_bounds__(256) loss_values_batch_kernel(const float2* __
 
 }  // namespace
 
-unsigned loss_blocks(uint32_t width, uint32_t height) {
-  return blocks_for((size_t)width * 3, kStrip) * blocks_for(height, kRowsPerBlock);
+unsigned loss_blocks(uint32_t width, uint32_t height, unsigned rows) {
+  return blocks_for((size_t)width * 3, kStrip) * blocks_for(height, rows);
+}
+
+unsigned loss_rows(const uint32_t* width, const uint32_t* height, size_t images) {
+  const auto fits = [&](unsigned rows) {
+    size_t blocks = 0;
+    for (size_t k = 0; k < images; k++) blocks += loss_blocks(width[k], height[k], rows);
+    return blocks <= kLossBlocks;
+  };
+  unsigned lo = kMinLossRows, hi = kMaxLossRows;  // the least that fits, or kMaxLossRows
+  while (lo < hi) {
+    const unsigned mid = (lo + hi) / 2;
+    if (fits(mid))
+      hi = mid;
+    else
+      lo = mid + 1;
+  }
+  return lo;
 }
 
 void loss_forward_backward_batch(splat_ctx* ctx, const float* pred, const BatchDev& bd,
-                                 unsigned total_blocks, size_t total_values, float lambda,
-                                 float* dimage, float* scratch, float* losses) {
+                                 unsigned total_blocks, unsigned rows, size_t total_values,
+                                 float lambda, float* dimage, float* scratch, float* losses) {
   Taps taps;
   gaussian_kernel_host(taps.k);
   const float c1 = 0.01f * 0.01f, c2 = 0.03f * 0.03f;
@@ -498,11 +523,11 @@ void loss_forward_backward_batch(splat_ctx* ctx, const float* pred, const BatchD
   float2* partial = reinterpret_cast<float2*>(scratch + 3 * total_values);
   launch(ctx, "loss_ssim_stats", ssim_stats_kernel<true, true>, dim3(total_blocks), dim3(256), 0,
          pred, (const void*)nullptr, 0u, 0u, taps, c1, c2, d_mu, d_exx, d_exy, partial,
-         (const StepDyn*)nullptr, bd);
+         (const StepDyn*)nullptr, bd, (int)rows);
   launch(ctx, "loss_grad", ssim_grad_kernel<true, 0, true>, dim3(total_blocks), dim3(256), 0,
          pred, (const void*)nullptr, 0u, 0u, taps, (const float*)d_mu, (const float*)d_exx,
          (const float*)d_exy, 0.0f, 0.0f, lambda, dimage, (const StepDyn*)nullptr, bd,
-         StepLossReport{});
+         StepLossReport{}, (int)rows);
   if (losses)
     launch(ctx, "loss_value", loss_values_batch_kernel, dim3(bd.npairs), dim3(256), 0,
            (const float2*)partial, bd, lambda, losses);
@@ -511,7 +536,7 @@ void loss_forward_backward_batch(splat_ctx* ctx, const float* pred, const BatchD
 void loss_value_to(splat_ctx* ctx, const float* scratch, uint32_t width, uint32_t height,
                    float lambda, float* out_dev, const StepDyn* dyn) {
   const size_t n = (size_t)width * height * 3;
-  const unsigned nb = blocks_for((size_t)width * 3, kStrip) * blocks_for(height, kRowsPerBlock);
+  const unsigned nb = loss_blocks(width, height, loss_rows(&width, &height, 1));
   launch(ctx, "loss_value", loss_value_kernel, dim3(1), dim3(256), 0,
          reinterpret_cast<const float2*>(scratch + 3 * n), nb, lambda, (float)n, out_dev, dyn);
 }
@@ -530,16 +555,17 @@ hipError_t loss_launch_bare(hipStream_t stream, const float* pred, const float* 
   float* d_exx = scratch + n;
   float* d_exy = scratch + 2 * n;
   float2* partial = reinterpret_cast<float2*>(scratch + 3 * n);
-  const dim3 grid(blocks_for((size_t)width * 3, kStrip), blocks_for(height, kRowsPerBlock));
+  const unsigned rows = loss_rows(&width, &height, 1);
+  const dim3 grid(blocks_for((size_t)width * 3, kStrip), blocks_for(height, rows));
   const float inv_n = 1.0f / (float)n;
   const float w1 = (1.0f - lambda) * inv_n;
   hipLaunchKernelGGL((ssim_stats_kernel<false, false>), grid, dim3(256), 0, stream, pred,
                      (const void*)target, width, height, taps, c1, c2, d_mu, d_exx, d_exy,
-                     partial, (const StepDyn*)nullptr, BatchDev{});
+                     partial, (const StepDyn*)nullptr, BatchDev{}, (int)rows);
   hipLaunchKernelGGL((ssim_grad_kernel<false, 0, false>), grid, dim3(256), 0, stream, pred,
                      (const void*)target, width, height, taps, (const float*)d_mu,
                      (const float*)d_exx, (const float*)d_exy, inv_n, w1, lambda, dimage,
-                     (const StepDyn*)nullptr, BatchDev{}, StepLossReport{});
+                     (const StepDyn*)nullptr, BatchDev{}, StepLossReport{}, (int)rows);
   if (loss_out)
     hipLaunchKernelGGL(loss_value_kernel, dim3(1), dim3(256), 0, stream,
                        (const float2*)partial, grid.x * grid.y, lambda, (float)n, loss_out,
@@ -561,8 +587,7 @@ void gaussian_kernel_host(float k[11]) {
 
 size_t loss_scratch_floats(uint32_t width, uint32_t height) {
   const size_t n = (size_t)width * height * 3;
-  const size_t blocks = (size_t)blocks_for(n / height, kStrip) * blocks_for(height, kRowsPerBlock);
-  return 3 * n + 2 * blocks + 64;
+  return 3 * n + 2 * (size_t)loss_blocks(width, height, loss_rows(&width, &height, 1)) + 64;
 }
 
 // Runs both passes.  target_u8 (trainer views) or target_f32 (host tier) must be given.
@@ -581,7 +606,8 @@ void loss_forward_backward(splat_ctx* ctx, const float* pred, const float* targe
   float* d_exx = scratch + n;
   float* d_exy = scratch + 2 * n;
   float2* partial = reinterpret_cast<float2*>(scratch + 3 * n);
-  const dim3 grid(blocks_for((size_t)width * 3, kStrip), blocks_for(height, kRowsPerBlock));
+  const unsigned rows = loss_rows(&width, &height, 1);
+  const dim3 grid(blocks_for((size_t)width * 3, kStrip), blocks_for(height, rows));
   const float inv_n = 1.0f / (float)n;
   const float w1 = (1.0f - lambda) * inv_n;
   StepLossReport rep{};
@@ -594,30 +620,32 @@ void loss_forward_backward(splat_ctx* ctx, const float* pred, const float* targe
   }
   if (target_u8) {
     launch(ctx, "loss_ssim_stats", ssim_stats_kernel<true, false>, grid, dim3(256), 0, pred,
-           (const void*)target_u8, width, height, taps, c1, c2, d_mu, d_exx, d_exy, partial, dyn, BatchDev{});
+           (const void*)target_u8, width, height, taps, c1, c2, d_mu, d_exx, d_exy, partial, dyn, BatchDev{},
+           (int)rows);
     if (want_l1)
       launch(ctx, "loss_grad", ssim_grad_kernel<true, 0, false>, grid, dim3(256), 0, pred,
              (const void*)target_u8, width, height, taps, (const float*)d_mu,
              (const float*)d_exx, (const float*)d_exy, inv_n, w1, lambda, dimage, dyn,
-             BatchDev{}, rep);
+             BatchDev{}, rep, (int)rows);
     else
       launch(ctx, "loss_grad", ssim_grad_kernel<true, 1, false>, grid, dim3(256), 0, pred,
              (const void*)target_u8, width, height, taps, (const float*)d_mu,
              (const float*)d_exx, (const float*)d_exy, inv_n, w1, lambda, dimage, dyn,
-             BatchDev{}, rep);
+             BatchDev{}, rep, (int)rows);
   } else {
     launch(ctx, "loss_ssim_stats", ssim_stats_kernel<false, false>, grid, dim3(256), 0, pred,
-           (const void*)target_f32, width, height, taps, c1, c2, d_mu, d_exx, d_exy, partial, dyn, BatchDev{});
+           (const void*)target_f32, width, height, taps, c1, c2, d_mu, d_exx, d_exy, partial, dyn, BatchDev{},
+           (int)rows);
     if (want_l1)
       launch(ctx, "loss_grad", ssim_grad_kernel<false, 0, false>, grid, dim3(256), 0, pred,
              (const void*)target_f32, width, height, taps, (const float*)d_mu,
              (const float*)d_exx, (const float*)d_exy, inv_n, w1, lambda, dimage, dyn,
-             BatchDev{}, rep);
+             BatchDev{}, rep, (int)rows);
     else
       launch(ctx, "loss_grad", ssim_grad_kernel<false, 1, false>, grid, dim3(256), 0, pred,
              (const void*)target_f32, width, height, taps, (const float*)d_mu,
              (const float*)d_exx, (const float*)d_exy, inv_n, w1, lambda, dimage, dyn,
-             BatchDev{}, rep);
+             BatchDev{}, rep, (int)rows);
   }
   if (loss_parts_host) {
     const size_t nb = (size_t)grid.x * grid.y;
