@@ -12,16 +12,19 @@
 //   4. scatter one 16-byte record per entry into its tile's bucket: the key (depth bits
 //      << 32 | entry) and the entry's Gaussian;
 //   5. sort each bucket by that 64-bit value, the Gaussian carried along: tiles of up to
-//      1024 entries by one wave each (a bitonic network in registers, lanes exchanging
-//      by DPP and the gfx950 row swaps), up to 16384 by a bitonic sort in LDS (1024-lane workgroups,
-//      128 KB), in global memory beyond.  This equals the reference's (key, entry) order.
+//      512 entries by one wave each (a bitonic network in registers, lanes exchanging
+//      by DPP and the gfx950 row swaps), larger ones by a workgroup of eight waves that sort
+//      runs and rank every entry in the other runs (in LDS up to 4096 entries; beyond,
+//      chunks of 4096 are ranked through global memory).  This equals the reference's (key, entry) order.
 #include "internal.hpp"
 
 namespace splat {
 namespace {
 
 constexpr int kWaveCap = 512;     // entries per tile sorted by one wave (8 per lane)
-constexpr int kMidCap = 1024;     // ... by one wave of the second kernel (16 per lane)
+constexpr uint32_t kRunWaves = 8;  // waves of the workgroups that sort larger tiles
+constexpr uint32_t kRunCap = 512 * kRunWaves;  // entries they sort in LDS (8 per lane)
+constexpr uint32_t kQueueFirst = 1024;  // tiles beyond this many entries are sorted first
 constexpr uint32_t kKeygenThreads = 256;
 constexpr uint32_t kKeygenPerLane = 1;
 constexpr uint32_t kKeygenEntries = kKeygenThreads * kKeygenPerLane;  // per keygen workgroup
@@ -30,7 +33,6 @@ constexpr uint32_t kKeygenEntries = kKeygenThreads * kKeygenPerLane;  // per key
 
 // Counter set of the keygen workgroup that handles entry e.
 __device__ __forceinline__ uint32_t entry_sub(uint32_t e) { return (e / kKeygenEntries) % kTileSub; }
-constexpr int kBigCap = 16384;    // entries per tile sorted in LDS by the 1024-lane kernel
 
 // Last g in [lo, hi) with off[g] <= e, given off[lo] <= e < off[hi] (Gaussians with zero
 // entries are skipped: they share their offset with the next Gaussian).
@@ -251,64 +253,6 @@ __global__ void guard_kernel(const unsigned long long* __restrict__ total64,
   if (t > capacity) status->abort = 1u;
 }
 
-// One bitonic step over `n` keys (virtual +inf padding beyond n).  Pairs p in [0, half).
-// `size` (>= 2) and `stride` are powers of two: shifts and masks index the pairs.
-template <class Load, class Store>
-__device__ __forceinline__ void bitonic_pairs(uint32_t n, uint32_t half, uint32_t size,
-                                              uint32_t stride, bool flip, Load ld, Store st) {
-  const uint32_t lh = (uint32_t)__builtin_ctz(size) - 1u;  // log2(size / 2)
-  const uint32_t ls = stride ? (uint32_t)__builtin_ctz(stride) : 0u;
-  for (uint32_t p = threadIdx.x; p < half; p += blockDim.x) {
-    uint32_t i, j;
-    if (flip) {
-      const uint32_t blk = p >> lh, off = p & ((1u << lh) - 1u);
-      i = (blk << (lh + 1u)) + off;
-      j = (blk << (lh + 1u)) + size - 1 - off;
-    } else {
-      i = ((p >> ls) << (ls + 1u)) + (p & (stride - 1u));
-      j = i + stride;
-    }
-    if (j < n) {
-      const uint64_t a = ld(i), b = ld(j);
-      if (a > b) {
-        st(i, b);
-        st(j, a);
-      }
-    }
-  }
-}
-
-__device__ __forceinline__ uint32_t next_pow2(uint32_t v) {
-  uint32_t p = 1;
-  while (p < v) p <<= 1;
-  return p;
-}
-
-template <class Load, class Store>
-__device__ void bitonic_sort(uint32_t n, Load ld, Store st) {
-  const uint32_t N = next_pow2(n);
-  const uint32_t half = N >> 1;
-  for (uint32_t size = 2; size <= N; size <<= 1) {
-    bitonic_pairs(n, half, size, 0, true, ld, st);
-    __syncthreads();
-    for (uint32_t stride = size >> 2; stride >= 1; stride >>= 1) {
-      bitonic_pairs(n, half, size, stride, false, ld, st);
-      __syncthreads();
-    }
-  }
-}
-
-__device__ __forceinline__ void write_sorted(uint32_t pos, uint64_t v, uint32_t tile,
-                                             const uint32_t* __restrict__ entry_gaussian,
-                                             uint32_t* __restrict__ sorted_entry,
-                                             uint32_t* __restrict__ sorted_gauss,
-                                             uint64_t* __restrict__ keys_out) {
-  const uint32_t entry = (uint32_t)v;
-  sorted_entry[pos] = entry;
-  sorted_gauss[pos] = entry_gaussian[entry];
-  if (keys_out) keys_out[pos] = ((uint64_t)tile << 32) | (v >> 32);
-}
-
 // ---- per-tile sorts in one wave ----------------------------------------------------
 // A tile of at most 64 K entries is sorted by one wave holding K (key, Gaussian) pairs per
 // lane in registers: a bitonic network over N = 64 K positions (padding keys all ones),
@@ -446,9 +390,9 @@ __device__ __forceinline__ void wave_sort_tile(uint32_t lane, uint32_t tile, uin
   }
 }
 
-// One wave per tile (four per workgroup).  Larger tiles are queued in `queue` (T words):
-// up to kMidCap entries from the end (count in *mid_count), beyond from the start (count
-// in *big_count); a tile is queued at most once, so the two never meet.
+// One wave per tile (four per workgroup).  Larger tiles are queued in `queue` (T words): those
+// beyond kQueueFirst entries from the start (count in counts[0]), the others from the end (count in
+// counts[2]); a tile is queued at most once, so the two never meet.
 __global__ void __launch_bounds__(256) sort_tiles_kernel(uint32_t num_tiles,
                                                          const uint32_t* __restrict__ tile_start,
                                                          const uint4* __restrict__ bucket,
@@ -456,8 +400,7 @@ __global__ void __launch_bounds__(256) sort_tiles_kernel(uint32_t num_tiles,
                                                          uint32_t* __restrict__ sorted_gauss,
                                                          uint64_t* __restrict__ keys_out,
                                                          uint32_t* __restrict__ queue,
-                                                         uint32_t* __restrict__ big_count,
-                                                         uint32_t* __restrict__ mid_count) {
+                                                         uint32_t* __restrict__ counts) {
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t tile = blockIdx.x * 4u + (threadIdx.x >> 6);
   if (tile >= num_tiles) return;
@@ -465,10 +408,10 @@ __global__ void __launch_bounds__(256) sort_tiles_kernel(uint32_t num_tiles,
   if (n == 0) return;
   if (n > (uint32_t)kWaveCap) {
     if (lane == 0) {
-      if (n > (uint32_t)kMidCap)
-        queue[atomicAdd(big_count, 1u)] = tile;
+      if (n > kQueueFirst)
+        queue[atomicAdd(&counts[0], 1u)] = tile;
       else
-        queue[num_tiles - 1 - atomicAdd(mid_count, 1u)] = tile;
+        queue[num_tiles - 1 - atomicAdd(&counts[2], 1u)] = tile;
     }
     return;
   }
@@ -482,63 +425,129 @@ __global__ void __launch_bounds__(256) sort_tiles_kernel(uint32_t num_tiles,
     wave_sort_tile<8>(lane, tile, s, n, bucket, sorted_entry, sorted_gauss, keys_out);
 }
 
-// The queued tiles of kWaveCap < n <= kMidCap entries, one wave each (the grid's waves
-// stride over the queue; a wave leaves when it is exhausted).
-__global__ void __launch_bounds__(256) sort_mid_kernel(uint32_t num_tiles,
-                                                       const uint32_t* __restrict__ tile_start,
-                                                       const uint4* __restrict__ bucket,
-                                                       uint32_t* __restrict__ sorted_entry,
-                                                       uint32_t* __restrict__ sorted_gauss,
-                                                       uint64_t* __restrict__ keys_out,
-                                                       const uint32_t* __restrict__ queue,
-                                                       const uint32_t* __restrict__ mid_count) {
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t count = *mid_count;
-  for (uint32_t q = blockIdx.x * 4u + (threadIdx.x >> 6); q < count; q += gridDim.x * 4u) {
-    const uint32_t tile = queue[num_tiles - 1 - q];
-    const uint32_t s = tile_start[tile], n = tile_start[tile + 1] - s;
-    wave_sort_tile<16>(lane, tile, s, n, bucket, sorted_entry, sorted_gauss, keys_out);
+// Sorts the n <= 64 K kRunWaves records at bucket[s ..]: each wave sorts a run of 64 K in
+// registers, the runs' keys go to LDS, and an entry's place is its place in its own run plus
+// the number of smaller keys in every other run (binary searches of 8 entries' worth of
+// independent chains at a time; keys are distinct).  put(place, key, Gaussian) takes the
+// entries.  Call from every lane; `sh` may be reused after a barrier.  (Merging neighbouring
+// runs pair by pair does a third of the searches, but their barriers and rewrites made the
+// launch slower, 58 against 45 us.)
+template <int K, class Put>
+__device__ __forceinline__ void run_sort(uint32_t s, uint32_t n, const uint4* bucket,
+                                         uint64_t* sh, Put&& put) {
+  constexpr uint32_t L = 64 * K;  // a run
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  uint64_t key[K];
+  uint32_t gid[K], place[K];
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    const uint32_t p = wave * L + (uint32_t)k * 64u + lane;
+    const uint4 r = p < n ? bucket[s + p] : make_uint4(~0u, ~0u, 0u, 0u);
+    key[k] = ((uint64_t)r.y << 32) | r.x;
+    gid[k] = r.z;
   }
+  wave_sort_stages<K, 2, 1>(key, gid, lane);
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    place[k] = lane * K + k;
+    sh[wave * L + place[k]] = key[k];
+  }
+  __syncthreads();
+  const uint32_t runs = (n + L - 1) / L;  // the others hold padding only
+  constexpr int R = K >= 8 ? 1 : 8 / K;   // runs searched side by side
+  for (uint32_t w0 = 0; w0 + 1 < runs; w0 += R) {
+    uint32_t base[R], pos[R][K];
+    bool on[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      // the w-th run but for the own one; a chain past the last run repeats it for nothing
+      const uint32_t w = w0 + r;
+      on[r] = w + 1 < runs;
+      const uint32_t q = min(w, runs - 2);
+      base[r] = (q < wave ? q : q + 1) * L;
+#pragma unroll
+      for (int k = 0; k < K; k++) pos[r][k] = 0;
+    }
+#pragma unroll
+    for (uint32_t step = L / 2; step >= 1; step >>= 1)
+#pragma unroll
+      for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int k = 0; k < K; k++)
+          pos[r][k] += sh[base[r] + pos[r][k] + step - 1] < key[k] ? step : 0u;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+      for (int k = 0; k < K; k++) {
+        const uint32_t below = pos[r][k] + (sh[base[r] + pos[r][k]] < key[k] ? 1u : 0u);
+        place[k] += on[r] ? below : 0u;
+      }
+  }
+#pragma unroll
+  for (int k = 0; k < K; k++)
+    if (key[k] != ~0ull) put(place[k], key[k], gid[k]);
 }
 
-// Queued tiles: LDS bitonic up to kBigCap entries, global-memory bitonic beyond.  The
-// grid strides over the queue; every workgroup exits once the queue is exhausted.
-__global__ void __launch_bounds__(1024) sort_big_kernel(const uint32_t* __restrict__ tile_start,
-                                                        uint4* __restrict__ bucket,
-                                                        const uint32_t* __restrict__ entry_gaussian,
-                                                        uint32_t* __restrict__ sorted_entry,
-                                                        uint32_t* __restrict__ sorted_gauss,
-                                                        uint64_t* __restrict__ keys_out,
-                                                        const uint32_t* __restrict__ big_list,
-                                                        const uint32_t* __restrict__ big_count) {
-  __shared__ uint64_t sh[kBigCap];
-  const uint32_t count = *big_count;
-  // the records' keys (their Gaussians come from entry_gaussian)
-  const auto rec_key = [&](uint32_t i) {
-    const uint2 k = *reinterpret_cast<const uint2*>(&bucket[i]);
-    return ((uint64_t)k.y << 32) | k.x;
-  };
+// The queued tiles (more than kWaveCap entries), one workgroup each; the grid strides over the
+// queue.  Bound by the latency of the networks and searches of the largest tiles.  At 300k
+// Gaussians, 1297x840 (1066 such tiles, 335 beyond 1024 entries, up to 3023), this took
+// 39 us where one wave per tile up to 1024 entries and a bitonic sort in LDS by 1024 lanes
+// beyond took 28 + 56 us; with a handful of tiles of 500-1000 entries 7 us
+// against 22 + 4, with none 6 us against 5 + 5.
+__global__ void __launch_bounds__(64 * kRunWaves, 4) sort_queue_kernel(
+    const uint32_t* __restrict__ tile_start, uint4* bucket, uint32_t* __restrict__ sorted_entry,
+    uint32_t* __restrict__ sorted_gauss, uint64_t* __restrict__ keys_out,
+    uint32_t num_tiles, const uint32_t* __restrict__ queue,
+    const uint32_t* __restrict__ counts) {
+  __shared__ uint64_t sh[kRunCap];
+  const uint32_t first = counts[0], count = first + counts[2];
   for (uint32_t q = blockIdx.x; q < count; q += gridDim.x) {
-    const uint32_t tile = big_list[q];
+    const uint32_t tile = queue[q < first ? q : num_tiles - 1 - (q - first)];
     const uint32_t s = tile_start[tile], n = tile_start[tile + 1] - s;
-    if (n <= kBigCap) {
-      for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) sh[i] = rec_key(s + i);
-      __syncthreads();
-      bitonic_sort(n, [&](uint32_t i) { return sh[i]; },
-                   [&](uint32_t i, uint64_t v) { sh[i] = v; });
-      for (uint32_t i = threadIdx.x; i < n; i += blockDim.x)
-        write_sorted(s + i, sh[i], tile, entry_gaussian, sorted_entry, sorted_gauss, keys_out);
+    const auto emit = [&](uint32_t place, uint64_t key, uint32_t gid) {
+      sorted_entry[s + place] = (uint32_t)key;
+      sorted_gauss[s + place] = gid;
+      if (keys_out) keys_out[s + place] = ((uint64_t)tile << 32) | (key >> 32);
+    };
+    if (n <= kRunCap / 4) {
+      run_sort<2>(s, n, bucket, sh, emit);
+    } else if (n <= kRunCap / 2) {
+      run_sort<4>(s, n, bucket, sh, emit);
+    } else if (n <= kRunCap) {
+      run_sort<8>(s, n, bucket, sh, emit);
     } else {
-      bitonic_sort(n, [&](uint32_t i) { return rec_key(s + i); },
-                   [&](uint32_t i, uint64_t v) {
-                     *reinterpret_cast<uint2*>(&bucket[s + i]) =
-                         make_uint2((uint32_t)v, (uint32_t)(v >> 32));
-                   });
-      for (uint32_t i = threadIdx.x; i < n; i += blockDim.x)
-        write_sorted(s + i, rec_key(s + i), tile, entry_gaussian, sorted_entry, sorted_gauss,
-                     keys_out);
+      // chunks sorted in place, then every entry ranked in the other chunks
+      for (uint32_t c = 0; c < n; c += kRunCap) {
+        run_sort<8>(s + c, min(kRunCap, n - c), bucket, sh,
+                    [&](uint32_t place, uint64_t key, uint32_t gid) {
+                      bucket[s + c + place] =
+                          make_uint4((uint32_t)key, (uint32_t)(key >> 32), gid, 0u);
+                    });
+        __syncthreads();
+      }
+      const auto key_at = [&](uint32_t i) {
+        const uint2 k = *reinterpret_cast<const uint2*>(&bucket[s + i]);
+        return ((uint64_t)k.y << 32) | k.x;
+      };
+      for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
+        const uint4 r = bucket[s + i];
+        const uint64_t key = ((uint64_t)r.y << 32) | r.x;
+        uint32_t place = i % kRunCap;
+        for (uint32_t c = 0; c < n; c += kRunCap) {
+          if (c == i / kRunCap * kRunCap) continue;
+          uint32_t lo = c, len = min(kRunCap, n - c);  // first entry of the chunk not below key
+          while (len > 0) {
+            const uint32_t half = len / 2;
+            const bool below = key_at(lo + half) < key;
+            lo = below ? lo + half + 1 : lo;
+            len = below ? len - half - 1 : half;
+          }
+          place += lo - c;
+        }
+        emit(place, key, r.z);
+      }
     }
-    __syncthreads();
+    __syncthreads();  // sh is free
   }
 }
 
@@ -869,21 +878,16 @@ void tile_layout(splat_ctx* ctx, const BinBuffers& bb, size_t T, uint32_t* total
   tile_order(ctx, bb, T);
 }
 
-// counts[0] (big tiles) and counts[2] (mid tiles) start at zero; `queue` holds T words.
+// counts[0] and counts[2] (queued tiles) start at zero; `queue` holds T words.
 void sort_tiles(splat_ctx* ctx, const BinBuffers& bb, size_t T, uint64_t* keys_out,
                 uint32_t* queue, uint32_t* counts) {
   launch(ctx, "bin_sort_tiles", sort_tiles_kernel, dim3(blocks_for(T, 4)), dim3(256), 0,
          (uint32_t)T, (const uint32_t*)bb.tile_start, (const uint4*)bb.bucket,
-         bb.sorted_entry, bb.sorted_gauss, keys_out, queue,
-         counts, counts + 2);
-  launch(ctx, "bin_sort_mid", sort_mid_kernel, dim3(512), dim3(256), 0, (uint32_t)T,
-         (const uint32_t*)bb.tile_start, (const uint4*)bb.bucket,
-         bb.sorted_entry, bb.sorted_gauss, keys_out,
-         (const uint32_t*)queue, (const uint32_t*)(counts + 2));
-  launch(ctx, "bin_sort_big", sort_big_kernel, dim3(256), dim3(1024), 0,
-         (const uint32_t*)bb.tile_start, bb.bucket, (const uint32_t*)bb.entry_gaussian,
-         bb.sorted_entry, bb.sorted_gauss, keys_out, (const uint32_t*)queue,
-         (const uint32_t*)counts);
+         bb.sorted_entry, bb.sorted_gauss, keys_out, queue, counts);
+  // two workgroups at a time per compute unit (16 waves of 128 VGPRs), two more in turn
+  launch(ctx, "bin_sort_queue", sort_queue_kernel, dim3((unsigned)std::min<size_t>(T, 1024)),
+         dim3(64 * kRunWaves), 0, (const uint32_t*)bb.tile_start, bb.bucket, bb.sorted_entry,
+         bb.sorted_gauss, keys_out, (uint32_t)T, (const uint32_t*)queue, (const uint32_t*)counts);
 }
 
 }  // namespace
@@ -899,7 +903,7 @@ size_t bin_build(splat_ctx* ctx, ProjBuffers pb, size_t n, uint32_t tiles_x, uin
   bb.tile_sub = (uint32_t*)store["tile_sub"].reserve((kTileSub + 1) * T * 4);
   bb.tile_start = (uint32_t*)store["tile_start"].reserve((T + 1) * 4);
   bb.tile_order = (uint32_t*)store["tile_order"].reserve(T * 4 + 4);
-  uint32_t* small = (uint32_t*)store["bin_small"].reserve(64);  // [0] E, [1] big count, [2] T
+  uint32_t* small = (uint32_t*)store["bin_small"].reserve(64);  // [0] E, [1] and [3] queued tiles, [2] T
   unsigned long long* total64 = (unsigned long long*)store["bin_total64"].reserve(8);
   uint32_t* big_list = (uint32_t*)store["bin_big_list"].reserve(T * 4);
 
