@@ -978,17 +978,11 @@ void bin_build_device(splat_ctx* ctx, ProjBuffers pb, size_t n, const BinBuffers
                       uint32_t* big_list, uint32_t* scan_sums, StepStatus* status,
                       const BatchDev* bd) {
   const size_t T = (size_t)bb.tiles_x * bb.tiles_y;
-  // the capacity guard and the keygen marks ride on the scan's last pass when it has one
+  // the capacity guard and the keygen marks ride on the scan
   const ScanTail tail{bb.block_marks, (uint32_t)(capacity / kKeygenEntries + 2), kKeygenEntries,
                       (unsigned long long)capacity, total64, status};
-  if (!exclusive_scan_u32(ctx, pb.ntiles, bb.entry_offset, n, small, scan_sums, total64,
-                          bd ? nullptr : &tail)) {
-    bin_guard(ctx, total64, capacity, status);
-    // The entry kernels cover the capacity and read the step's count from `status`.
-    launch(ctx, "bin_marks", block_marks_kernel<>, dim3(blocks_for(n, 256)), dim3(256), 0,
-           (const uint32_t*)bb.entry_offset, (uint32_t)n, bb.block_marks,
-           (const StepStatus*)status);
-  }
+  exclusive_scan_u32(ctx, pb.ntiles, bb.entry_offset, n, small, scan_sums, total64, &tail);
+  // The entry kernels cover the capacity and read the step's count from `status`.
   if (bd)
     launch(ctx, "bin_keygen", keygen_batch_kernel, dim3(blocks_for(capacity, kKeygenEntries)),
            dim3(kKeygenThreads), 0, (const uint32_t*)bb.entry_offset, (uint32_t)n, *bd,

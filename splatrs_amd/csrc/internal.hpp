@@ -451,7 +451,7 @@ void planes_to_aos(splat_ctx* ctx, const float* planes, size_t n, size_t stride,
 // `sums` (scan_temp_bytes(n) bytes) defaults to a context scratch buffer; graph-captured
 // code passes its own so the captured pointer stays valid.  `total64` (optional, zeroed by
 // the caller) receives the exact 64-bit sum of the input.
-// Extra work of the last pass of the entry-offset scan of a graph-captured step: the
+// Extra work of the entry-offset scan of a graph-captured step (in its last pass): the
 // capacity guard (total64 against `capacity`, into `status`) and the keygen marks.
 struct ScanTail {
   uint32_t* marks;
@@ -460,9 +460,7 @@ struct ScanTail {
   const unsigned long long* total64;
   StepStatus* status;
 };
-// Returns whether `tail` was done (only by the multi-pass scan, n > scan_single's limit;
-// the caller does it otherwise).
-bool exclusive_scan_u32(splat_ctx* ctx, const uint32_t* in, uint32_t* out, size_t n,
+void exclusive_scan_u32(splat_ctx* ctx, const uint32_t* in, uint32_t* out, size_t n,
                         uint32_t* total_dev, uint32_t* sums = nullptr,
                         unsigned long long* total64 = nullptr, const ScanTail* tail = nullptr);
 size_t scan_temp_bytes(size_t n);
