@@ -672,8 +672,8 @@ __global__ void __launch_bounds__(256) project_bwd_kernel(const float* __restric
 // the float4 gradient of plane j, rows r..r+3.  kU groups per lane are in flight: their
 // parameter and moment loads are issued together, before any of their updates (one group's
 // 48 bytes per lane between waits leaves HBM latency exposed at a few waves per SIMD).
-// Groups that run past `rows` take the scalar path.  `ib` and `stride` are multiples of 64.
-template <uint32_t R, typename GradFn>
+// Groups that run past `rows` take the scalar path.  `ib` is a multiple of 4, `stride` of 64.
+template <uint32_t R, uint32_t THREADS, typename GradFn>
 __device__ __forceinline__ void adam_groups(float* __restrict__ params, float* __restrict__ m,
                                             float* __restrict__ v, uint32_t stride, uint32_t ib,
                                             uint32_t rows, const splat_learning_rates& lr,
@@ -682,14 +682,14 @@ __device__ __forceinline__ void adam_groups(float* __restrict__ params, float* _
   constexpr uint32_t kPerPlane = R / 4;  // float4 groups per plane
   constexpr uint32_t kGroups = kParams * kPerPlane;
   constexpr uint32_t kU = 4;
-  for (uint32_t q0 = threadIdx.x; q0 < kGroups; q0 += kU * R) {
+  for (uint32_t q0 = threadIdx.x; q0 < kGroups; q0 += kU * THREADS) {
     float4 P[kU], M[kU], V[kU];
 #pragma unroll
     for (uint32_t u = 0; u < kU; u++) {
       // unconditional, so the loads issue back to back: a group past the rows (used by the
       // scalar path or not at all) reads rows ib..ib+3 of plane 0 instead, which exist since
-      // ib < n <= stride and both ib and stride are multiples of 64
-      const uint32_t q = q0 + u * R;
+      // ib < n <= stride and both ib and stride are multiples of 4
+      const uint32_t q = q0 + u * THREADS;
       const uint32_t j = q / kPerPlane, r = (q % kPerPlane) * 4u;
       const size_t at = q < kGroups && r + 4 <= rows ? (size_t)j * stride + ib + r : (size_t)ib;
       // the parameter planes are read and written with ordinary (cached) accesses: the
@@ -701,7 +701,7 @@ __device__ __forceinline__ void adam_groups(float* __restrict__ params, float* _
     }
 #pragma unroll
     for (uint32_t u = 0; u < kU; u++) {
-      const uint32_t q = q0 + u * R;
+      const uint32_t q = q0 + u * THREADS;
       const uint32_t j = q / kPerPlane, r = (q % kPerPlane) * 4u;
       if (q >= kGroups || r >= rows) continue;
       const float rate = plane_lr((int)j, lr);
@@ -738,22 +738,28 @@ __device__ __forceinline__ void adam_groups(float* __restrict__ params, float* _
 // dc * basis, the product project_backward_one takes.  The arithmetic is that of the
 // separate host-tier kernels (a plane without a term gets a zero gradient of either sign,
 // which Adam treats alike).
-constexpr uint32_t kGradAdamRows = 128;  // Gaussian rows per grad_adam workgroup
+//
+// R rows and THREADS lanes per workgroup: 128 and 128 stream large models.  A model of up to
+// kGradAdamSmall rows gets too few such workgroups to fill the chip, and each of them takes its
+// 1888 float4 groups in four rounds of 16 loads per lane; with 64 rows and 256 lanes (the first
+// 64 run the projection backward) there are twice as many workgroups and one round: 31 -> 20 us
+// at 10k rows, 53 -> 44 at 61k (300k: 109 -> 143, 1M: 287 -> 387, which keep the large form).
+constexpr uint32_t kGradAdamRows = 128, kGradAdamRowsSmall = 64, kGradAdamSmall = 1u << 16;
 constexpr uint32_t kGradWords = 11 + 16 + 3;  // LDS words per row: planes 0-10, basis, dc
 
-__global__ void __launch_bounds__(kGradAdamRows) grad_adam_kernel(
+template <uint32_t R, uint32_t THREADS>
+__global__ void __launch_bounds__(THREADS) grad_adam_kernel(
     float* __restrict__ params, float* __restrict__ m, float* __restrict__ v, uint32_t n,
     uint32_t stride, CameraDev cam, float near_plane, float eps2d, int antialias, int degree,
     const uint32_t* __restrict__ entry_offset, const float* __restrict__ slots, StatsArgs sa,
     float c1, float c2, float b1, float b2, float eps, splat_learning_rates lr,
     const StepDyn* __restrict__ dyn, const StepStatus* __restrict__ status) {
-  constexpr uint32_t R = kGradAdamRows;
   constexpr uint32_t kChunk = 2 * R;  // entries staged per pass
   constexpr uint32_t kShared =
       kChunk * kSlots > kGradWords * R ? kChunk * kSlots : kGradWords * R;
   __shared__ __align__(16) float sh[kShared];
   if (status && status->abort) return;  // uniform: every lane reads the same flag
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = threadIdx.x < R ? blockIdx.x * R + threadIdx.x : 0xffffffffu;  // this lane's row
   if (dyn) {
     cam = dyn->cam;
     c1 = dyn->c1;
@@ -763,7 +769,7 @@ __global__ void __launch_bounds__(kGradAdamRows) grad_adam_kernel(
   float sum[kSlots];
 #pragma unroll
   for (int k = 0; k < kSlots; k++) sum[k] = 0.0f;
-  const uint32_t ib = blockIdx.x * blockDim.x, ie = min(ib + blockDim.x, n);
+  const uint32_t ib = blockIdx.x * R, ie = min(ib + R, n);
   const uint32_t span0 = entry_offset[ib], span1 = entry_offset[ie];
   const uint32_t e0 = i < n ? entry_offset[i] : 0u, e1 = i < n ? entry_offset[i + 1] : 0u;
   // words per entry: the backward writes the absolute sums (slots 9, 10) exactly when the
@@ -773,20 +779,21 @@ __global__ void __launch_bounds__(kGradAdamRows) grad_adam_kernel(
   for (uint32_t c0 = span0; c0 < span1; c0 += kChunk) {
     const uint32_t c1e = min(c0 + kChunk, span1);
     __syncthreads();
-    {  // 16 coalesced loads per lane in flight before their LDS stores
-      constexpr uint32_t kLoads = 16;
+    {  // up to 16 coalesced loads per lane in flight before their LDS stores
+      constexpr uint32_t kAll = (kChunk * 9 + THREADS - 1) / THREADS;
+      constexpr uint32_t kLoads = kAll < 16 ? kAll : 16;
       const uint32_t words = (c1e - c0) * ns;
       const float* src = slots + (size_t)c0 * ns;
-      for (uint32_t q0 = threadIdx.x; q0 < words; q0 += kLoads * R) {
+      for (uint32_t q0 = threadIdx.x; q0 < words; q0 += kLoads * THREADS) {
         float x[kLoads];
 #pragma unroll
         for (uint32_t u = 0; u < kLoads; u++) {
-          const uint32_t q = q0 + u * R;
+          const uint32_t q = q0 + u * THREADS;
           x[u] = src[min(q, words - 1)];  // in the span: no branch between the loads
         }
 #pragma unroll
         for (uint32_t u = 0; u < kLoads; u++) {
-          const uint32_t q = q0 + u * R;
+          const uint32_t q = q0 + u * THREADS;
           if (q < words) sh[q] = x[u];
         }
       }
@@ -804,8 +811,10 @@ __global__ void __launch_bounds__(kGradAdamRows) grad_adam_kernel(
   }
   __syncthreads();  // the staging buffer now holds gradients
   float* const gw = sh + threadIdx.x;  // this row's column: word w at gw[w * R]
+  if (threadIdx.x < R) {
 #pragma unroll
-  for (uint32_t w = 0; w < kGradWords; w++) gw[w * R] = 0.0f;
+    for (uint32_t w = 0; w < kGradWords; w++) gw[w * R] = 0.0f;
+  }
   if (i < n) {
   splat_proj_grad pg;
   pg.mean2d[0] = sum[0];
@@ -847,14 +856,14 @@ __global__ void __launch_bounds__(kGradAdamRows) grad_adam_kernel(
                      });
   }
   __syncthreads();  // every row's gradient words are in LDS
-  adam_groups<R>(params, m, v, stride, ib, ie - ib, lr, b1, b2, c1, c2, eps,
-                 [&](uint32_t j, uint32_t r) {
-                   if (j < 11) return *reinterpret_cast<const float4*>(sh + j * R + r);
-                   const uint32_t kk = (j - 11) / 3, ch = (j - 11) % 3;
-                   const float4 dc = *reinterpret_cast<const float4*>(sh + (27 + ch) * R + r);
-                   const float4 bs = *reinterpret_cast<const float4*>(sh + (11 + kk) * R + r);
-                   return make_float4(dc.x * bs.x, dc.y * bs.y, dc.z * bs.z, dc.w * bs.w);
-                 });
+  adam_groups<R, THREADS>(
+      params, m, v, stride, ib, ie - ib, lr, b1, b2, c1, c2, eps, [&](uint32_t j, uint32_t r) {
+        if (j < 11) return *reinterpret_cast<const float4*>(sh + j * R + r);
+        const uint32_t kk = (j - 11) / 3, ch = (j - 11) % 3;
+        const float4 dc = *reinterpret_cast<const float4*>(sh + (27 + ch) * R + r);
+        const float4 bs = *reinterpret_cast<const float4*>(sh + (11 + kk) * R + r);
+        return make_float4(dc.x * bs.x, dc.y * bs.y, dc.z * bs.z, dc.w * bs.w);
+      });
 }
 
 // Batched backward tail and optimizer, one wave of 64 scene rows per workgroup (scene rows
@@ -905,7 +914,7 @@ __global__ void __launch_bounds__(kBatchRows) grad_adam_batch_kernel(
   }
   __syncthreads();
   lr.mean = bd.lr_mean[s];
-  adam_groups<R>(params, m, v, stride, ib, rows, lr, b1, b2, c1, c2, eps,
+  adam_groups<R, R>(params, m, v, stride, ib, rows, lr, b1, b2, c1, c2, eps,
                  [&](uint32_t j, uint32_t r) {
                    return *reinterpret_cast<const float4*>(acc + j * R + r);
                  });
@@ -977,11 +986,16 @@ void grad_adam(splat_ctx* ctx, float* params, float* m, float* v, size_t n, size
                const float* slots, const StatsArgs& sa, float c1, float c2,
                const splat_adam_state& st, const splat_learning_rates& lr, const StepDyn* dyn,
                const StepStatus* status) {
-  launch(ctx, "grad_adam", grad_adam_kernel, dim3(blocks_for(n, kGradAdamRows)),
-         dim3(kGradAdamRows), 0, params, m,
-         v, (uint32_t)n, (uint32_t)stride, camera_dev(cam), opts.near_plane, opts.eps2d,
-         opts.antialias, opts.sh_degree, entry_offset, slots, sa, c1, c2, st.beta1, st.beta2,
-         st.eps, lr, dyn, status);
+  const auto go = [&](auto kernel, uint32_t rows, uint32_t threads) {
+    launch(ctx, "grad_adam", kernel, dim3(blocks_for(n, rows)), dim3(threads), 0, params, m, v,
+           (uint32_t)n, (uint32_t)stride, camera_dev(cam), opts.near_plane, opts.eps2d,
+           opts.antialias, opts.sh_degree, entry_offset, slots, sa, c1, c2, st.beta1, st.beta2,
+           st.eps, lr, dyn, status);
+  };
+  if (n <= kGradAdamSmall)
+    go(grad_adam_kernel<kGradAdamRowsSmall, 256>, kGradAdamRowsSmall, 256);
+  else
+    go(grad_adam_kernel<kGradAdamRows, kGradAdamRows>, kGradAdamRows, kGradAdamRows);
 }
 
 void project_forward_batch(splat_ctx* ctx, const float* params, size_t stride,
