@@ -27,8 +27,8 @@ namespace {
 // 140, 4293 tiles 502 / 363; FEW with 32-entry batches lies between at all four sizes.
 constexpr unsigned kFewTilesFwd = 6144;
 constexpr unsigned kFewTilesBwd = 1536;
+constexpr unsigned kFewTilesOrd = 768;  // ordered backward, see raster_bwd_ordered_kernel
 constexpr int kOrdBatch = 32;      // entries staged per batch (ordered backward)
-constexpr uint32_t kOrdTerms = 1024;  // pixel terms per slot staged at a time (a tile has 256)
 
 struct TileInfo {
   uint32_t gx0, gy0, w, h;
@@ -406,8 +406,9 @@ struct PixBack {
 // Returns whether any lane of the wave contributes; v[] holds the slot terms (zero for
 // lanes that do not), and the pixel state advances only on contributing lanes.  The
 // reference's expressions and correctly rounded divisions: the ordered backward is bitwise.
+// bg (uniform over the wave): the background term is not a zero for every lane.
 __device__ __forceinline__ bool pair_terms(PixBack& s, bool act, float4 r0, float4 r1, float4 r2,
-                                           float px, float py, const uint64_t* tab,
+                                           float px, float py, const uint64_t* tab, bool bg,
                                            float v[kSlots]) {
 #pragma unroll
   for (int q = 0; q < kSlots; q++) v[q] = 0.0f;
@@ -430,7 +431,8 @@ __device__ __forceinline__ bool pair_terms(PixBack& s, bool act, float4 r0, floa
   dalpha += (r2.z - a1) * s.d1;
   dalpha += (r2.w - a2) * s.d2;
   dalpha *= t;
-  dalpha += (-s.t_final / (1.0f - alpha)) * s.bg_dot;
+  // without a background the term is a zero, whose addition no sum sees
+  if (bg) dalpha += (-s.t_final / (1.0f - alpha)) * s.bg_dot;
   const bool p3 = p2 & (og < kAlphaMax);
   const float dgauss = o * dalpha;
   const float dsigma = -dgauss * G;
@@ -891,8 +893,20 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
 // entries of a group, as many as fit kOrdTerms pixels, lie one after the other, and a lane
 // sums one slot of one entry over the entry's own pixels.  Only the waves whose 8x8 block the
 // rectangle reaches evaluate it.
-template <bool ABS, bool BATCH, bool PERSIST>
-__global__ void __launch_bounds__(256) raster_bwd_ordered_kernel(
+//
+// FEW (launches with few tiles, kFewTilesOrd): bound by the latency of the walk and of the
+// sums' chains of up to 256 additions, so they overlap: a fifth wave sums a group while the
+// four of the pixels walk the next one into the other half of the staging, and loads the next
+// batch's records; a group holds four full tiles.  Otherwise the chip is filled by other
+// workgroups, walk and sums take turns and the staging is kept small (two full tiles).  In us,
+// FEW / otherwise / all 256 pixels of 8 entries staged at a time, as it was: 130 tiles of a
+// grown model (most entries cover their tiles) 511 / 680 / 1279, 256 tiles 177 / 229 / 403,
+// 1271 tiles 337 / 250 / 767, 4293 tiles 2060 / 875 / 4526, 8160 tiles 2401 / 750 / 5785.  (The
+// slots' rows lie four words apart modulo the LDS banks and are read 16 bytes at a time, the
+// next ones beside the additions; in step and one word at a time it was 940 at 130 tiles and
+// 1217 at 8160.)
+template <bool ABS, bool BATCH, bool PERSIST, bool FEW>
+__global__ void __launch_bounds__(FEW ? 320 : 256) raster_bwd_ordered_kernel(
     const float4* __restrict__ rec, const uint32_t* __restrict__ tile_start,
     const uint32_t* __restrict__ order,
     const uint32_t* __restrict__ sorted_gauss, const uint32_t* __restrict__ sorted_entry,
@@ -902,16 +916,21 @@ __global__ void __launch_bounds__(256) raster_bwd_ordered_kernel(
     uint32_t* __restrict__ counter) {
   constexpr uint32_t SS = ABS ? kSlots : 9;
   constexpr int B = kOrdBatch;
-  static_assert(B <= 64 && kOrdTerms >= 256, "one wave scans a batch; a group holds an entry");
+  constexpr uint32_t kTerms = FEW ? 1024 : 512;  // pixel terms per slot staged at a time
+  constexpr uint32_t kRow = kTerms + 4;          // words per slot: slots apart in the LDS banks
+  static_assert(B < 64 && kTerms >= 256, "one wave scans a batch; a group holds an entry");
+  // FEW: two batches and two groups, one being walked, the other summed or loaded
+  constexpr int kHalves = FEW ? 2 : 1;
   __shared__ uint64_t tab[32];
-  __shared__ float4 s0[B], s1[B], s2[B];
-  __shared__ uint32_t srect[B];
-  __shared__ uint32_t spre[B + 1];  // pixels of the batch entries before each one
+  __shared__ float4 s0[kHalves][B], s1[kHalves][B], s2[kHalves][B];
+  __shared__ uint32_t srect[kHalves][B], sentry[kHalves][B];
+  __shared__ uint32_t spre[kHalves][B + 1];  // staging words of the batch entries before each one
   __shared__ uint32_t smax_last;
   __shared__ uint32_t s_tile;
-  __shared__ float terms[SS * kOrdTerms];
+  __shared__ __align__(16) float terms[kHalves][SS * kRow + 16];  // (a sum reads 16 words ahead)
   if (threadIdx.x < 32) tab[threadIdx.x] = kExp2Table[threadIdx.x];
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool walker = !FEW || wave < 4;  // uniform over the wave
   for (;;) {
   const uint32_t tile = next_tile<PERSIST>(counter, &s_tile, order, num_tiles);
   if (tile >= num_tiles) break;
@@ -919,11 +938,13 @@ __global__ void __launch_bounds__(256) raster_bwd_ordered_kernel(
   const TileGeom tg = tile_geom<BATCH>(tile, tiles_x, W, H, bd);
   const TileInfo ti = tg.ti;
   uint32_t i, j;
-  tile_pixel(threadIdx.x, &i, &j);
-  const bool valid = i < ti.w && j < ti.h;
+  tile_pixel(threadIdx.x & 255u, &i, &j);
+  const bool valid = walker && i < ti.w && j < ti.h;
   const float px = (float)(ti.gx0 + i) + 0.5f;
   const float py = (float)(ti.gy0 + j) + 0.5f;
   PixBack s = pixel_back(tg, i, j, valid, bg0, bg1, bg2, final_t, n_contrib, dimage);
+  // whether the background term of some pixel of the wave is not a zero
+  const bool bg = __any(!(s.bg_dot == 0.0f) || !(fabsf(s.t_final) < INFINITY));
   const uint32_t start = tile_start[tile], end = tile_start[tile + 1];
   const uint32_t count = end - start;
   __syncthreads();
@@ -935,66 +956,124 @@ __global__ void __launch_bounds__(256) raster_bwd_ordered_kernel(
     const uint32_t k = q / SS;
     slots[(size_t)sorted_entry[start + k] * SS + q % SS] = 0.0f;
   }
+  // (one wave) the batch of entries [lo, lo + cnt) into half `h`
+  const auto stage = [&](uint32_t h, uint32_t lo, uint32_t cnt) {
+    uint32_t area = 0;
+    if (lane < cnt) {
+      const uint32_t at = start + lo + lane;
+      const StagedRecord r = load_record(rec, sorted_gauss[at]);
+      sentry[h][lane] = sorted_entry[at];
+      s0[h][lane] = half_conic0(r.a);
+      s1[h][lane] = half_conic1(r.b);
+      s2[h][lane] = r.c;
+      const uint32_t rc = entry_rect(r.a, r.b, r.c, ti);
+      srect[h][lane] = rc;
+      // whole groups of four, for 16-byte reads
+      area = ((uint32_t)__popc(rc & 0xffffu) * (uint32_t)__popc(rc >> 16) + 3u) & ~3u;
+    }
+    uint32_t pre = area;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t o = (uint32_t)__shfl_up((int)pre, d, 64);
+      if (lane >= (uint32_t)d) pre += o;
+    }
+    if (lane <= cnt) spre[h][lane] = pre - area;
+  };
+  // (lanes q0, q0 + step, ...) the slots of group [g0, g1) of the batch in half `h`, staged in
+  // terms[tb]
+  const auto sum_group = [&](uint32_t h, uint32_t g0, uint32_t g1, uint32_t tb, uint32_t q0,
+                             uint32_t step) {
+    const uint32_t p0 = spre[h][g0];
+    for (uint32_t q = q0; q < (g1 - g0) * SS; q += step) {
+      const uint32_t kk = g0 + q / SS, slot = q % SS;
+      const uint32_t rc = srect[h][kk];
+      const uint32_t n = (uint32_t)__popc(rc & 0xffffu) * (uint32_t)__popc(rc >> 16);
+      const float4* p =
+          reinterpret_cast<const float4*>(&terms[tb][slot * kRow + (spre[h][kk] - p0)]);
+      // the additions stay in order; the next eight terms are read beside them
+      float acc = 0.0f;
+      float4 x = p[0], y = p[1];  // (within the array whatever n is)
+      uint32_t t = 0;
+      for (; t + 8 <= n; t += 8) {
+        const float4 x0 = x, y0 = y;
+        x = p[t / 4 + 2];
+        y = p[t / 4 + 3];
+        acc += x0.x;
+        acc += x0.y;
+        acc += x0.z;
+        acc += x0.w;
+        acc += y0.x;
+        acc += y0.y;
+        acc += y0.z;
+        acc += y0.w;
+      }
+      const float rest[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+      for (uint32_t u = 0; u < 7; u++)
+        if (t + u < n) acc += rest[u];
+      slots[(size_t)sentry[h][kk] * SS + slot] = acc;
+    }
+  };
+  uint32_t h = 0, tb = 0;                        // batch half, staging half
+  uint32_t last_h = 0, last_g0 = 0, last_g1 = 0;  // the group walked before this one (none: g1 = 0)
+  if (FEW) {
+    if (!walker && kmax > 0) stage(0, max((int32_t)kmax - B, 0), min(kmax, (uint32_t)B));
+    __syncthreads();
+  }
   for (int32_t hi = (int32_t)kmax; hi > 0; hi -= B) {
     const int32_t lo = max(hi - B, 0);
     const uint32_t cnt = (uint32_t)(hi - lo);
-    __syncthreads();
-    if (threadIdx.x < 64) {
-      uint32_t area = 0;
-      if (threadIdx.x < cnt) {
-        const uint32_t g = sorted_gauss[start + lo + threadIdx.x];
-        const float4 a = rec[4 * g], b = rec[4 * g + 1], c = rec[4 * g + 2];
-        s0[threadIdx.x] = half_conic0(a);
-        s1[threadIdx.x] = half_conic1(b);
-        s2[threadIdx.x] = c;
-        const uint32_t rc = entry_rect(a, b, c, ti);
-        srect[threadIdx.x] = rc;
-        area = (uint32_t)__popc(rc & 0xffffu) * (uint32_t)__popc(rc >> 16);
-      }
-      uint32_t pre = area;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = (uint32_t)__shfl_up((int)pre, d, 64);
-        if (lane >= (uint32_t)d) pre += o;
-      }
-      if (lane <= cnt && lane <= (uint32_t)B) spre[lane] = pre - area;
+    if (!FEW) {
+      __syncthreads();
+      if (wave == 0) stage(0, (uint32_t)lo, cnt);
+      __syncthreads();
     }
-    __syncthreads();
     // groups of entries from the back, each the longest that fits the staging
-    const uint32_t my_pre = spre[min(lane, cnt)];
+    const uint32_t my_pre = spre[h][min(lane, cnt)];
     for (uint32_t g1 = cnt; g1 > 0;) {
-      const uint32_t p1 = spre[g1];
-      const uint64_t fits = __ballot(lane < g1 && p1 - my_pre <= kOrdTerms);
+      const uint32_t p1 = spre[h][g1];
+      const uint64_t fits = __ballot(lane < g1 && p1 - my_pre <= kTerms);
       const uint32_t g0 = (uint32_t)__builtin_ctzll(fits);  // entry g1 - 1 fits (<= 256 pixels)
-      const uint32_t p0 = spre[g0];
-      uint64_t todo = __ballot(lane >= g0 && lane < g1 && wave_touches(srect[min(lane, cnt - 1)], wave));
-      while (todo) {
-        const uint32_t kk = 63u - (uint32_t)__builtin_clzll(todo);
-        todo &= ~(1ull << kk);
-        const uint32_t rc = srect[kk];
-        const bool in = in_rect(rc, i, j);  // columns and rows are within the image
-        float v[kSlots];
-        pair_terms(s, valid & (lo + kk < s.last) & in, s0[kk], s1[kk], s2[kk], px, py, tab, v);
-        if (in) {
-          const uint32_t x0 = (uint32_t)__builtin_ctz(rc), y0 = (uint32_t)__builtin_ctz(rc >> 16);
-          const uint32_t pos = spre[kk] - p0 + (j - y0) * (uint32_t)__popc(rc & 0xffffu) + (i - x0);
+      if (walker) {
+        const uint32_t p0 = spre[h][g0];
+        uint64_t todo = __ballot(lane >= g0 && lane < g1 &&
+                                 wave_touches(srect[h][min(lane, cnt - 1)], wave));
+        while (todo) {
+          const uint32_t kk = 63u - (uint32_t)__builtin_clzll(todo);
+          todo &= ~(1ull << kk);
+          const uint32_t rc = srect[h][kk];
+          const bool in = in_rect(rc, i, j);  // columns and rows are within the image
+          float v[kSlots];
+          pair_terms(s, valid & (lo + kk < s.last) & in, s0[h][kk], s1[h][kk], s2[h][kk], px, py,
+                     tab, bg, v);
+          if (in) {
+            const uint32_t x0 = (uint32_t)__builtin_ctz(rc), y0 = (uint32_t)__builtin_ctz(rc >> 16);
+            const uint32_t pos =
+                spre[h][kk] - p0 + (j - y0) * (uint32_t)__popc(rc & 0xffffu) + (i - x0);
 #pragma unroll
-          for (int q = 0; q < (int)SS; q++) terms[q * kOrdTerms + pos] = v[q];
+            for (int q = 0; q < (int)SS; q++) terms[tb][q * kRow + pos] = v[q];
+          }
         }
+      } else {
+        if (last_g1) sum_group(last_h, last_g0, last_g1, tb ^ 1u, lane, 64);
+        // the other half's batch is summed: the next batch goes there, once per batch
+        if (g1 == cnt && lo > 0) stage(h ^ 1u, (uint32_t)max(lo - B, 0), min((uint32_t)lo, (uint32_t)B));
       }
       __syncthreads();
-      for (uint32_t q = threadIdx.x; q < (g1 - g0) * SS; q += blockDim.x) {
-        const uint32_t kk = g0 + q / SS, slot = q % SS;
-        const uint32_t n = spre[kk + 1] - spre[kk];
-        const float* p = &terms[slot * kOrdTerms + (spre[kk] - p0)];
-        float acc = 0.0f;
-        for (uint32_t t = 0; t < n; t++) acc += p[t];
-        slots[(size_t)sorted_entry[start + lo + kk] * SS + slot] = acc;
+      if (FEW) {
+        last_h = h;
+        last_g0 = g0;
+        last_g1 = g1;
+        tb ^= 1u;
+      } else {
+        sum_group(0, g0, g1, 0, threadIdx.x, 256);
+        __syncthreads();
       }
-      __syncthreads();
       g1 = g0;
     }
+    if (FEW) h ^= 1u;
   }
+  if (FEW && !walker && last_g1) sum_group(last_h, last_g0, last_g1, tb ^ 1u, lane, 64);
   if (!PERSIST) break;
   }
 }
@@ -1119,11 +1198,17 @@ void bwd_ordered_go(splat_ctx* ctx, const ProjBuffers& pb, const BinBuffers& bb,
                     const BatchDev& bd, uint32_t* counter, unsigned per_cu) {
   if (PERSIST) fill_u32(ctx, counter, kXcds, 0u);
   const unsigned grid = PERSIST ? persistent_grid(ctx, per_cu, T) : T;
-  launch(ctx, "raster_bwd_ordered", raster_bwd_ordered_kernel<ABS, BATCH, PERSIST>, dim3(grid),
-         dim3(256), 0, (const float4*)pb.rec, (const uint32_t*)bb.tile_start,
-         (const uint32_t*)bb.tile_order, (const uint32_t*)bb.sorted_gauss,
-         (const uint32_t*)bb.sorted_entry, T, bb.tiles_x, width,
-         height, bg[0], bg[1], bg[2], final_t, n_contrib, dimage, slots, bd, counter);
+  const auto go = [&](auto kernel, unsigned threads) {
+    launch(ctx, "raster_bwd_ordered", kernel, dim3(grid), dim3(threads), 0,
+           (const float4*)pb.rec, (const uint32_t*)bb.tile_start, (const uint32_t*)bb.tile_order,
+           (const uint32_t*)bb.sorted_gauss, (const uint32_t*)bb.sorted_entry, T, bb.tiles_x,
+           width, height, bg[0], bg[1], bg[2], final_t, n_contrib, dimage, slots, bd, counter);
+  };
+  if constexpr (!BATCH && !PERSIST) {
+    if (T <= kFewTilesOrd)
+      return go(raster_bwd_ordered_kernel<ABS, false, false, true>, 320);
+  }
+  go(raster_bwd_ordered_kernel<ABS, BATCH, PERSIST, false>, 256);
 }
 
 template <bool BATCH, bool PERSIST>
