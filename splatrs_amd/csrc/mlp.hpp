@@ -21,10 +21,12 @@ unsigned mlp_grad_rows(size_t count);
 void mlp_grad(splat_ctx* ctx, const void* packed, const float* params, const float* feats,
               const uint8_t* labels, const float* weights, const uint32_t* order, size_t count,
               float inv_batch, float* partial, float* partial_loss);
-// Sum of the partial rows (in row order) -> grad_out (optional); Adam on the master weights
-// when `update`.
-void mlp_reduce_update(splat_ctx* ctx, float* params, float* m, float* v, const float* partial,
-                       unsigned rows, float* grad_out, bool update, float lr, float c1, float c2);
-void mlp_loss_sum(splat_ctx* ctx, const float* partial_loss, unsigned rows, float* out);
+// Sums of the partial rows (in row order) -> grad_out (optional) and of the partial losses ->
+// loss_out; when `update`, Adam on the master weights and their packed operands, which mlp_pack
+// has written before.
+void mlp_reduce_update(splat_ctx* ctx, float* params, float* m, float* v, void* packed,
+                       const float* partial, const float* partial_loss, unsigned rows,
+                       float* grad_out, float* loss_out, bool update, float lr, float c1,
+                       float c2);
 
 }  // namespace splat

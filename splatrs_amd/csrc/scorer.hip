@@ -60,10 +60,9 @@ float scorer_fit_device(splat_scorer* s, const float* feats, const uint8_t* labe
       s->adam_step++;
       const float c1 = 1.0f - powi(0.9f, (int32_t)s->adam_step);
       const float c2 = 1.0f - powi(0.999f, (int32_t)s->adam_step);
-      mlp_reduce_update(ctx, s->params.as<float>(), s->m.as<float>(), s->v.as<float>(), partial,
-                        rows, nullptr, true, cfg.lr, c1, c2);
-      mlp_pack(ctx, s->params.as<float>(), s->packed.ptr);
-      mlp_loss_sum(ctx, ploss, rows, losses + nb);
+      mlp_reduce_update(ctx, s->params.as<float>(), s->m.as<float>(), s->v.as<float>(),
+                        s->packed.ptr, partial, ploss, rows, nullptr, losses + nb, true, cfg.lr,
+                        c1, c2);
     }
     std::vector<float> lv(nb);
     SPLAT_HIP(hipMemcpyAsync(lv.data(), losses, nb * 4, hipMemcpyDeviceToHost, ctx->stream));
@@ -181,9 +180,9 @@ int splat_scorer_loss_grad(splat_scorer* s, const float* features, const uint8_t
     SPLAT_HIP(hipMemcpyAsync(w, weights, n * 4, hipMemcpyHostToDevice, ctx->stream));
     mlp_grad(ctx, s->packed.ptr, s->params.as<float>(), f, y, w, nullptr, n, 1.0f / (float)n,
              partial, ploss);
-    mlp_reduce_update(ctx, s->params.as<float>(), s->m.as<float>(), s->v.as<float>(), partial,
-                      rows, g, false, 0.0f, 1.0f, 1.0f);
-    mlp_loss_sum(ctx, ploss, rows, g + kMlpParams);
+    mlp_reduce_update(ctx, s->params.as<float>(), s->m.as<float>(), s->v.as<float>(),
+                      s->packed.ptr, partial, ploss, rows, g, g + kMlpParams, false, 0.0f, 1.0f,
+                      1.0f);
     SPLAT_HIP(hipMemcpyAsync(grad, g, kMlpParams * 4, hipMemcpyDeviceToHost, ctx->stream));
     SPLAT_HIP(hipMemcpyAsync(loss, g + kMlpParams, 4, hipMemcpyDeviceToHost, ctx->stream));
     SPLAT_HIP(hipStreamSynchronize(ctx->stream));
