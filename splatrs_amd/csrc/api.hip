@@ -55,9 +55,8 @@ float* upload_planes(splat_ctx* ctx, const char* name, const float* aos, size_t 
 }
 
 void download_planes(splat_ctx* ctx, const float* planes, size_t n, size_t stride, float* aos) {
-  float* staging = ctx->buf<float>("aos_staging_out", n * kParams + 1);
-  planes_to_aos(ctx, planes, n, stride, staging);
-  d2h(ctx, aos, staging, n * kParams * 4);
+  const HostRecords array = {planes, n, stride, aos};
+  planes_to_host(ctx, &array, 1);
 }
 
 ProjBuffers alloc_proj(splat_ctx* ctx, size_t n) {

@@ -543,17 +543,11 @@ int splat_batch_download(splat_batch* b, uint32_t scene, float* gaussians, float
     const BatchScene& sc = b->scenes[scene];
     SPLAT_REQUIRE(capacity >= sc.n, "output capacity too small");
     splat_ctx* ctx = b->ctx;
-    float* staging = (float*)b->store["aos_out"].reserve(sc.n * kParams * 4);
-    const std::pair<float*, const DevBuf*> arrays[3] = {{gaussians, &b->params}, {m, &b->m},
-                                                        {v, &b->v}};
-    for (auto& a : arrays) {
-      if (!a.first) continue;
-      planes_to_aos(ctx, a.second->as<float>() + sc.off, sc.n, b->stride, staging);
-      SPLAT_HIP(hipMemcpyAsync(a.first, staging, sc.n * kParams * 4, hipMemcpyDeviceToHost,
-                               ctx->stream));
-      SPLAT_HIP(hipStreamSynchronize(ctx->stream));
-    }
-    b->store.erase("aos_out");
+    const HostRecords arrays[3] = {
+        {b->params.as<float>() + sc.off, sc.n, b->stride, gaussians},
+        {b->m.as<float>() + sc.off, sc.n, b->stride, m},
+        {b->v.as<float>() + sc.off, sc.n, b->stride, v}};
+    planes_to_host(ctx, arrays, 3);
   });
 }
 

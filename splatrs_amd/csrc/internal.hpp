@@ -85,6 +85,20 @@ struct DevBuf {
   }
 };
 
+// Pinned memory that models pass through on their way to the host (planes_to_host): 12 MB, taken
+// at a context's first such call and given back with the context.
+constexpr size_t kHostRingSlots = 12;
+struct HostRing {
+  void* ptr = nullptr;
+  hipEvent_t ready[kHostRingSlots] = {};
+  HostRing() = default;
+  HostRing(const HostRing&) = delete;
+  HostRing& operator=(const HostRing&) = delete;
+  ~HostRing();
+  void reserve();
+  float* slot(size_t k) const;
+};
+
 struct KernelStat {
   uint64_t launches = 0;
   double ms = 0;
@@ -107,6 +121,7 @@ struct splat_ctx {
   std::vector<hipEvent_t> event_pool;
   std::map<std::string, splat::KernelStat> kstats;
   std::map<std::string, splat::DevBuf> ws;  // named scratch buffers of the host tier
+  splat::HostRing ring;
 
   template <class T>
   T* buf(const char* name, size_t count) {
@@ -446,6 +461,13 @@ void grad_adam_batch(splat_ctx* ctx, float* params, float* m, float* v, size_t s
                      const uint32_t* entry_offset, const splat_proj_grad* dproj,
                      const splat_adam_state& st, const StepDyn* dyn, const StepStatus* status);
 void planes_to_aos(splat_ctx* ctx, const float* planes, size_t n, size_t stride, float* aos);
+// The records of several models (null `out`: none) in host memory, complete on return.
+struct HostRecords {
+  const float* planes;
+  size_t n, stride;
+  float* out;
+};
+void planes_to_host(splat_ctx* ctx, const HostRecords* arrays, size_t count);
 
 // scan.hip
 // `sums` (scan_temp_bytes(n) bytes) defaults to a context scratch buffer; graph-captured

@@ -997,16 +997,10 @@ int splat_trainer_download(splat_trainer* t, float* gaussians, float* m, float* 
     splat_ctx* ctx = t->ctx;
     const size_t n = t->n;
     if (n == 0) return;
-    float* staging = (float*)t->store["aos_out"].reserve(n * kParams * 4);
-    const std::pair<float*, const DevBuf*> arrays[3] = {{gaussians, &t->params}, {m, &t->m},
-                                                        {v, &t->v}};
-    for (auto& a : arrays) {
-      if (!a.first) continue;
-      planes_to_aos(ctx, a.second->as<float>(), n, t->stride, staging);
-      SPLAT_HIP(hipMemcpyAsync(a.first, staging, n * kParams * 4, hipMemcpyDeviceToHost,
-                               ctx->stream));
-      SPLAT_HIP(hipStreamSynchronize(ctx->stream));
-    }
+    const HostRecords arrays[3] = {{t->params.as<float>(), n, t->stride, gaussians},
+                                   {t->m.as<float>(), n, t->stride, m},
+                                   {t->v.as<float>(), n, t->stride, v}};
+    planes_to_host(ctx, arrays, 3);
     if (grad_accum)
       SPLAT_HIP(hipMemcpyAsync(grad_accum, t->grad_accum.ptr, n * 4, hipMemcpyDeviceToHost,
                                ctx->stream));
@@ -1016,7 +1010,6 @@ int splat_trainer_download(splat_trainer* t, float* gaussians, float* m, float* 
       SPLAT_HIP(hipMemcpyAsync(max_radii, t->max_radii.ptr, n * 4, hipMemcpyDeviceToHost,
                                ctx->stream));
     SPLAT_HIP(hipStreamSynchronize(ctx->stream));
-    t->store.erase("aos_out");
   });
 }
 
