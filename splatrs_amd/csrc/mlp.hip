@@ -12,7 +12,7 @@
 // units the lane holds, and the weight operands are packed in the same permuted order.
 //
 // Weight gradients contract over samples, so the error signals and activations of a
-// 64-sample chunk are staged in LDS transposed ([unit][sample]) and multiplied there; a
+// 32-sample chunk are staged in LDS transposed ([unit][sample]) and multiplied there; a
 // constant-one input turns the bias gradients into one more output column.
 //
 // Parameter layout (binary32 master copy): W1[64][12] b1[64] W2[64][64] b2[64] W3[64][64]
@@ -34,10 +34,11 @@ constexpr int kW1 = 0, kB1 = 768, kW2 = 832, kB2 = 4928, kW3 = 4992, kB3 = 9088,
 // layers 4, 3, 2 (4x1, 4x2, 4x2).
 constexpr int kF1 = 0, kF2 = 4, kF3 = 12, kF4 = 20, kT4 = 22, kT3 = 26, kT2 = 34,
               kBlocks = 42;
-constexpr int kChunk = 64;  // samples per workgroup pass of the training kernel
-// bfloat16 values between the LDS rows of two units: 144 bytes, so that the 16 rows which a
-// matrix operand is read from, 16 bytes each, lie in different banks (128 bytes: all in the same)
+constexpr int kChunk = 32;  // samples per workgroup pass of the training kernel
+// bfloat16 values between the LDS rows of two units: 80 bytes, so that the 16 rows which a
+// matrix operand is read from, 16 bytes each, lie in different banks
 constexpr int kRow = kChunk + 8;
+constexpr int kGradThreads = 512;
 
 __device__ __forceinline__ __bf16 to_bf16(float x) {  // round to nearest, ties to even
   uint32_t u = __float_as_uint(x);
@@ -142,63 +143,40 @@ __device__ __forceinline__ const T* reload(const T* p) {
   return p;
 }
 
-struct Fwd {
-  f32x4 z4;                   // logits (D layout, rows 0..2 in lanes 0..15)
-  f32x4 d1[4], d2[4], d3[4];  // GELU derivatives
-};
+__device__ __forceinline__ f32x4 gelu4(f32x4 z, const uint64_t* tab, f32x4* d) {
+  f32x4 a;
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    float dg;
+    a[r] = gelu(z[r], tab, &dg);
+    (*d)[r] = dg;
+  }
+  return a;
+}
 
-// `keep(layer, a)` is given each hidden layer's activations (binary32, rounded when used).
-template <class Keep>
-__device__ __forceinline__ void forward16(const bf16x8* __restrict__ packed,
-                                          const float* __restrict__ p, bf16x8 x, int lane,
-                                          const uint64_t* tab, Fwd& F, Keep&& keep) {
-  f32x4 a[4];
+// Logits (D layout, rows 0..2 in lanes 0..15) of a wave's 16 samples.
+__device__ __forceinline__ f32x4 forward16(const bf16x8* __restrict__ packed,
+                                           const float* __restrict__ p, bf16x8 x, int lane,
+                                           const uint64_t* tab) {
   const int g = lane >> 4;
+  f32x4 a[4], d;
 #pragma unroll
-  for (int mb = 0; mb < 4; mb++) {
-    const f32x4 z = mfma(blockop(packed, kF1 + mb, lane), x, bias4(p + kB1, mb, g));
+  for (int mb = 0; mb < 4; mb++)
+    a[mb] = gelu4(mfma(blockop(packed, kF1 + mb, lane), x, bias4(p + kB1, mb, g)), tab, &d);
 #pragma unroll
-    for (int r = 0; r < 4; r++) {
-      float d;
-      a[mb][r] = gelu(z[r], tab, &d);
-      F.d1[mb][r] = d;
+  for (int layer = 2; layer <= 3; layer++) {
+    const int f = layer == 2 ? kF2 : kF3, bias = layer == 2 ? kB2 : kB3;
+    const bf16x8 b0 = b_from_d(a, 0), b1 = b_from_d(a, 1);
+#pragma unroll
+    for (int mb = 0; mb < 4; mb++) {
+      f32x4 z = bias4(p + bias, mb, g);
+      z = mfma(blockop(packed, f + 2 * mb, lane), b0, z);
+      a[mb] = gelu4(mfma(blockop(packed, f + 2 * mb + 1, lane), b1, z), tab, &d);
     }
   }
-  bf16x8 b0 = b_from_d(a, 0), b1 = b_from_d(a, 1);
-  keep(1, a);
-#pragma unroll
-  for (int mb = 0; mb < 4; mb++) {
-    f32x4 z = bias4(p + kB2, mb, g);
-    z = mfma(blockop(packed, kF2 + 2 * mb, lane), b0, z);
-    z = mfma(blockop(packed, kF2 + 2 * mb + 1, lane), b1, z);
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      float d;
-      a[mb][r] = gelu(z[r], tab, &d);
-      F.d2[mb][r] = d;
-    }
-  }
-  b0 = b_from_d(a, 0);
-  b1 = b_from_d(a, 1);
-  keep(2, a);
-#pragma unroll
-  for (int mb = 0; mb < 4; mb++) {
-    f32x4 z = bias4(p + kB3, mb, g);
-    z = mfma(blockop(packed, kF3 + 2 * mb, lane), b0, z);
-    z = mfma(blockop(packed, kF3 + 2 * mb + 1, lane), b1, z);
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      float d;
-      a[mb][r] = gelu(z[r], tab, &d);
-      F.d3[mb][r] = d;
-    }
-  }
-  b0 = b_from_d(a, 0);
-  b1 = b_from_d(a, 1);
-  keep(3, a);
-  f32x4 acc = bias_d(p + kB4, kOut, 0, g);
-  acc = mfma(blockop(packed, kF4, lane), b0, acc);
-  F.z4 = mfma(blockop(packed, kF4 + 1, lane), b1, acc);
+  f32x4 z = bias_d(p + kB4, kOut, 0, g);
+  z = mfma(blockop(packed, kF4, lane), b_from_d(a, 0), z);
+  return mfma(blockop(packed, kF4 + 1, lane), b_from_d(a, 1), z);
 }
 
 // Packs the binary32 master weights into the bfloat16 operand blocks.
@@ -249,7 +227,7 @@ __global__ void __launch_bounds__(256) mlp_pack_kernel(const float* __restrict__
 
 // Logits of n feature rows ([n][12] -> [n][3]); one wave per 16 samples, grid-stride.  Bound by
 // the vector instructions of the activations: 93 us at 300k rows (135 us with branches in the
-// exponential and every layer's operands held in registers).
+// exponential and all operands held in registers).
 __global__ void __launch_bounds__(256) mlp_forward_kernel(const bf16x8* __restrict__ packed,
                                                           const float* __restrict__ p,
                                                           const float* __restrict__ feats,
@@ -265,11 +243,10 @@ __global__ void __launch_bounds__(256) mlp_forward_kernel(const bf16x8* __restri
     float f[kIn];
 #pragma unroll
     for (int k = 0; k < kIn; k++) f[k] = s < n ? feats[(size_t)s * kIn + k] : 0.0f;
-    Fwd F;
-    forward16(reload(packed), reload(p), feature_operand(f, g), lane, tab, F, [](int, const f32x4*) {});
+    const f32x4 z = forward16(reload(packed), reload(p), feature_operand(f, g), lane, tab);
     if (g == 0 && s < n) {
 #pragma unroll
-      for (int o = 0; o < kOut; o++) logits[(size_t)s * kOut + o] = F.z4[o];
+      for (int o = 0; o < kOut; o++) logits[(size_t)s * kOut + o] = z[o];
     }
   }
 }
@@ -278,38 +255,25 @@ __device__ __forceinline__ float softplus(float z) {
   return z > 0.0f ? z + log1pf(splat_expf(-z)) : log1pf(splat_expf(z));
 }
 
-// Stage D-layout values (MBLOCKS M-blocks) of one wave's 16 samples into an LDS [unit][sample]
-// array.
-template <int MBLOCKS>
-__device__ __forceinline__ void stage(uint16_t* s, const f32x4* v, int lane, int wave) {
-  const int g = lane >> 4, col = 16 * wave + (lane & 15);
-#pragma unroll
-  for (int mb = 0; mb < MBLOCKS; mb++)
-#pragma unroll
-    for (int r = 0; r < 4; r++) s[(16 * mb + 4 * g + r) * kRow + col] = bf16_bits(v[mb][r]);
+// bfloat16 D values of one M-block, as half a B operand of the next layer: units
+// 16 mb + 4g .. + 3 of the lane's sample.
+__device__ __forceinline__ uint2 pack4(f32x4 v) {
+  return make_uint2(bf16_bits(v[0]) | (uint32_t)bf16_bits(v[1]) << 16,
+                    bf16_bits(v[2]) | (uint32_t)bf16_bits(v[3]) << 16);
 }
 
-// The operand of 16 units over staged samples 32 kb .. 32 kb + 31.
-__device__ __forceinline__ bf16x8 staged(const uint16_t* s, int mb, int kb, int lane) {
-  return *reinterpret_cast<const bf16x8*>(s + (16 * mb + (lane & 15)) * kRow + 32 * kb +
-                                          8 * (lane >> 4));
+// Stage one M-block of one wave's 16 samples (D layout, packed) into an LDS [unit][sample] array.
+__device__ __forceinline__ void stage(uint16_t* s, uint2 v, int mb, int lane, int group) {
+  uint16_t* at = s + (16 * mb + 4 * (lane >> 4)) * kRow + 16 * group + (lane & 15);
+  at[0] = (uint16_t)v.x;
+  at[kRow] = (uint16_t)(v.x >> 16);
+  at[2 * kRow] = (uint16_t)v.y;
+  at[3 * kRow] = (uint16_t)(v.y >> 16);
 }
 
-// Weight-gradient tiles of one wave over the staged samples: row block mb, column blocks
-// nb0 .. nb0 + N - 1 and, with BIAS, one of the constant-one input.
-template <int N, bool BIAS>
-__device__ __forceinline__ void wgrad(const uint16_t* sE, const uint16_t* sA, int mb, int nb0,
-                                      int lane, f32x4* acc) {
-  const __bf16 one = (lane & 15) == 0 ? __builtin_bit_cast(__bf16, (uint16_t)0x3F80)
-                                      : __builtin_bit_cast(__bf16, (uint16_t)0);
-  const bf16x8 ones = {one, one, one, one, one, one, one, one};
-#pragma unroll
-  for (int kb = 0; kb < 2; kb++) {
-    const bf16x8 e = staged(sE, mb, kb, lane);
-#pragma unroll
-    for (int k = 0; k < N; k++) acc[k] = mfma(e, staged(sA, nb0 + k, kb, lane), acc[k]);
-    if (BIAS) acc[N] = mfma(e, ones, acc[N]);
-  }
+// The operand of 16 units over the staged samples.
+__device__ __forceinline__ bf16x8 staged(const uint16_t* s, int mb, int lane) {
+  return *reinterpret_cast<const bf16x8*>(s + (16 * mb + (lane & 15)) * kRow + 8 * (lane >> 4));
 }
 
 // Write a 16x16 tile of weight gradients (row block mb, column block nb; `nin` columns are
@@ -331,13 +295,17 @@ __device__ __forceinline__ void write_tile(float* __restrict__ row, int wbase, i
 // Gradient of the weighted binary cross-entropy over `count` samples (ids order[0..count)
 // or 0..count), scaled by inv_batch.  Each workgroup accumulates its chunks' weight
 // gradients in registers and writes one partial gradient row (kMlpParams floats) plus its
-// partial loss; mlp_adam_kernel sums the rows in workgroup order.  At a batch of 4096, 64
-// workgroups of one chunk: bound by the latency of that chunk's seven layers.  All layers are
-// staged in LDS of their own, so that one barrier separates the samples' part (a wave has 16
-// samples) from the weights' part (a wave has row block `wave` of layers 3 to 1 and column
-// block `wave` of layer 4): 31.7 us with rows of 128 bytes and two barriers per layer, 22.5 us
-// now, most of it the vector instructions of a wave's 48 activations per lane.
-__global__ void __launch_bounds__(256) mlp_grad_kernel(
+// partial loss; mlp_adam_kernel sums the rows.
+//
+// Wave w has sample group w % 2 (16 samples) and M-block w / 2 (16 units) of every hidden layer:
+// a layer's values are exchanged through LDS, where the weight gradients find them too (row
+// block w / 2 of layers 3 and 1 on the even waves, of layer 2 on the odd ones, and layer 4's
+// column block w / 2).  Bound by the
+// chain of seven layers, mostly the vector instructions of the activations: a wave has 12 per
+// lane.  A batch of 4096 makes 128 workgroups, 15.2 us; 64 workgroups of four waves with 48
+// activations per lane took 22.5 us, and 31.7 us with two barriers per layer and LDS rows of
+// 128 bytes, all in the same banks.
+__global__ void __launch_bounds__(kGradThreads) mlp_grad_kernel(
     const bf16x8* __restrict__ packed, const float* __restrict__ p,
     const float* __restrict__ feats, const uint8_t* __restrict__ labels,
     const float* __restrict__ weights, const uint32_t* __restrict__ order, uint32_t count,
@@ -346,107 +314,124 @@ __global__ void __launch_bounds__(256) mlp_grad_kernel(
   __shared__ __attribute__((aligned(16))) uint16_t sE4[16 * kRow], sE3[64 * kRow],
       sE2[64 * kRow], sE1[64 * kRow], sA3[64 * kRow], sA2[64 * kRow], sA1[64 * kRow],
       sX[16 * kRow];
-  __shared__ float sloss[4];
+  __shared__ uint2 exch[5][2][4][64];  // activations 1 to 3, errors 3 and 2; group, M-block, lane
+  __shared__ float sloss[2];
   __shared__ uint64_t tab[32];
   load_exp_table(tab);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4;
-  f32x4 acc[13];  // layer 4: column block `wave`, bias; layers 3 and 2: 4 and bias; layer 1
+  const int group = wave & 1, mb = wave >> 1;
+  // four column blocks and the bias of layer 3 (even waves) or 2; layer 1 (even) or layer 4 and
+  // its bias
+  f32x4 acc[7];
 #pragma unroll
-  for (int k = 0; k < 13; k++) acc[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int k = 0; k < 7; k++) acc[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const __bf16 one = (lane & 15) == 0 ? __builtin_bit_cast(__bf16, (uint16_t)0x3F80)
+                                      : __builtin_bit_cast(__bf16, (uint16_t)0);
+  const bf16x8 ones = {one, one, one, one, one, one, one, one};  // the constant-one input
+  // hand a layer's values on: the whole group's as the next layer's two B operands
+  const auto exchange = [&](int slot, uint2 v, bf16x8* b0, bf16x8* b1) {
+    exch[slot][group][mb][lane] = v;
+    __syncthreads();
+    const uint2 u0 = exch[slot][group][0][lane], u1 = exch[slot][group][1][lane],
+                u2 = exch[slot][group][2][lane], u3 = exch[slot][group][3][lane];
+    *b0 = __builtin_bit_cast(bf16x8, make_uint4(u0.x, u0.y, u1.x, u1.y));
+    *b1 = __builtin_bit_cast(bf16x8, make_uint4(u2.x, u2.y, u3.x, u3.y));
+  };
   float lsum = 0.0f;
   const uint32_t chunks = (count + kChunk - 1) / kChunk;
   for (uint32_t ch = blockIdx.x; ch < chunks; ch += gridDim.x) {
-    const uint32_t idx = ch * kChunk + 16 * wave + (lane & 15);
+    const uint32_t idx = ch * kChunk + 16 * group + (lane & 15);
     const bool valid = idx < count;
     const uint32_t s = valid ? (order ? order[idx] : idx) : 0;
     float f[kIn];
 #pragma unroll
     for (int k = 0; k < kIn; k++) f[k] = valid ? feats[(size_t)s * kIn + k] : 0.0f;
-    const bf16x8 x = feature_operand(f, g);
-    Fwd F;
-    forward16(reload(packed), reload(p), x, lane, tab, F, [&](int layer, const f32x4* a) {
-      stage<4>(layer == 1 ? sA1 : layer == 2 ? sA2 : sA3, a, lane, wave);
-    });
-    // output error (rows 0..2 live in lanes g == 0)
-    f32x4 e4 = {0.0f, 0.0f, 0.0f, 0.0f};
     const float w = valid ? weights[s] : 0.0f;
     const uint32_t y = valid ? labels[s] : 0u;
+    const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 d1, d2, d3;
+    bf16x8 b0, b1;
+    uint2 v = pack4(gelu4(mfma(blockop(packed, kF1 + mb, lane), feature_operand(f, g),
+                               bias4(p + kB1, mb, g)),
+                          tab, &d1));
+    stage(sA1, v, mb, lane, group);
+    exchange(0, v, &b0, &b1);
+    f32x4 z = mfma(blockop(packed, kF2 + 2 * mb, lane), b0, bias4(p + kB2, mb, g));
+    v = pack4(gelu4(mfma(blockop(packed, kF2 + 2 * mb + 1, lane), b1, z), tab, &d2));
+    stage(sA2, v, mb, lane, group);
+    exchange(1, v, &b0, &b1);
+    z = mfma(blockop(packed, kF3 + 2 * mb, lane), b0, bias4(p + kB3, mb, g));
+    v = pack4(gelu4(mfma(blockop(packed, kF3 + 2 * mb + 1, lane), b1, z), tab, &d3));
+    stage(sA3, v, mb, lane, group);
+    exchange(2, v, &b0, &b1);
+    z = mfma(blockop(packed, kF4, lane), b0, bias_d(p + kB4, kOut, 0, g));
+    z = mfma(blockop(packed, kF4 + 1, lane), b1, z);
+    // output error (rows 0..2 live in lanes g == 0), on each of the group's waves
+    f32x4 e4 = none;
     if (g == 0 && valid) {
 #pragma unroll
       for (int o = 0; o < kOut; o++) {
-        const float z = F.z4[o];
         const float yo = (y >> o) & 1u ? 1.0f : 0.0f;
-        lsum += w * (softplus(z) - yo * z) * inv_batch;
-        const float sg = 1.0f / (1.0f + splat_expf(-z));
+        if (mb == 0) lsum += w * (softplus(z[o]) - yo * z[o]) * inv_batch;
+        const float sg = 1.0f / (1.0f + expf_clamp(-z[o], tab));
         e4[o] = w * (sg - yo) * inv_batch;
       }
     }
-    // round the error signal as the matrix-core operand will see it
-#pragma unroll
-    for (int r = 0; r < 4; r++) e4[r] = __builtin_bit_cast(float, (uint32_t)bf16_bits(e4[r]) << 16);
-    bf16x8 E;
-#pragma unroll
-    for (int q = 0; q < 8; q++) E[q] = to_bf16(q < 4 ? e4[q] : 0.0f);
-    const bf16x8* back = reload(packed);
-    f32x4 e3[4], e2[4], e1[4];
-#pragma unroll
-    for (int mb = 0; mb < 4; mb++) {
-      const f32x4 t = mfma(blockop(back, kT4 + mb, lane), E, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-#pragma unroll
-      for (int r = 0; r < 4; r++) e3[mb][r] = t[r] * F.d3[mb][r];
-    }
-    bf16x8 E0 = b_from_d(e3, 0), E1 = b_from_d(e3, 1);
-#pragma unroll
-    for (int mb = 0; mb < 4; mb++) {
-      f32x4 t = mfma(blockop(back, kT3 + 2 * mb, lane), E0, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-      t = mfma(blockop(back, kT3 + 2 * mb + 1, lane), E1, t);
-#pragma unroll
-      for (int r = 0; r < 4; r++) e2[mb][r] = t[r] * F.d2[mb][r];
-    }
-    E0 = b_from_d(e2, 0);
-    E1 = b_from_d(e2, 1);
-#pragma unroll
-    for (int mb = 0; mb < 4; mb++) {
-      f32x4 t = mfma(blockop(back, kT2 + 2 * mb, lane), E0, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-      t = mfma(blockop(back, kT2 + 2 * mb + 1, lane), E1, t);
-#pragma unroll
-      for (int r = 0; r < 4; r++) e1[mb][r] = t[r] * F.d1[mb][r];
-    }
-    stage<1>(sE4, &e4, lane, wave);
-    stage<4>(sE3, e3, lane, wave);
-    stage<4>(sE2, e2, lane, wave);
-    stage<4>(sE1, e1, lane, wave);
-    if (g < 2) {
+    v = pack4(e4);
+    if (mb == 0) stage(sE4, v, 0, lane, group);
+    const bf16x8 E = __builtin_bit_cast(bf16x8, make_uint4(v.x, v.y, 0u, 0u));
+    v = pack4(mfma(blockop(packed, kT4 + mb, lane), E, none) * d3);
+    stage(sE3, v, mb, lane, group);
+    exchange(3, v, &b0, &b1);
+    z = mfma(blockop(packed, kT3 + 2 * mb, lane), b0, none);
+    v = pack4(mfma(blockop(packed, kT3 + 2 * mb + 1, lane), b1, z) * d2);
+    stage(sE2, v, mb, lane, group);
+    exchange(4, v, &b0, &b1);
+    z = mfma(blockop(packed, kT2 + 2 * mb, lane), b0, none);
+    v = pack4(mfma(blockop(packed, kT2 + 2 * mb + 1, lane), b1, z) * d1);
+    stage(sE1, v, mb, lane, group);
+    if (mb == 0 && g < 2) {
 #pragma unroll
       for (int q = 0; q < 8; q++) {
         const int k = 8 * g + q;
-        const float v = k < kIn ? f[k] : (k == kIn ? 1.0f : 0.0f);
-        sX[k * kRow + 16 * wave + (lane & 15)] = bf16_bits(v);
+        const float x = k < kIn ? f[k] : 0.0f;
+        sX[k * kRow + 16 * group + (lane & 15)] = k == kIn ? 0x3F80 : bf16_bits(x);
       }
     }
     __syncthreads();
-    wgrad<1, true>(sE4, sA3, 0, wave, lane, acc);
-    wgrad<4, true>(sE3, sA2, wave, 0, lane, acc + 2);
-    wgrad<4, true>(sE2, sA1, wave, 0, lane, acc + 7);
-    wgrad<1, false>(sE1, sX, wave, 0, lane, acc + 12);
+    const uint16_t *se = group ? sE2 : sE3, *sa = group ? sA1 : sA2;
+    const bf16x8 e = staged(se, mb, lane);
+#pragma unroll
+    for (int nb = 0; nb < 4; nb++) acc[nb] = mfma(e, staged(sa, nb, lane), acc[nb]);
+    acc[4] = mfma(e, ones, acc[4]);
+    if (group) {
+      const bf16x8 e4b = staged(sE4, 0, lane);
+      acc[5] = mfma(e4b, staged(sA3, mb, lane), acc[5]);
+      acc[6] = mfma(e4b, ones, acc[6]);
+    } else {
+      acc[5] = mfma(staged(sE1, mb, lane), staged(sX, 0, lane), acc[5]);
+    }
     __syncthreads();
   }
   // write this workgroup's gradient row
   float* row = partial + (size_t)blockIdx.x * kMlpParams;
-  write_tile(row, kW4, kB4, kHid, kOut, 0, wave, lane, acc[0]);
-  if (wave == 0) write_tile(row, kW4, kB4, kHid, kOut, 0, 4, lane, acc[1]);
+  const int wbase = group ? kW2 : kW3, bbase = group ? kB2 : kB3;
 #pragma unroll
-  for (int nb = 0; nb < 5; nb++) {
-    write_tile(row, kW3, kB3, kHid, kHid, wave, nb, lane, acc[2 + nb]);
-    write_tile(row, kW2, kB2, kHid, kHid, wave, nb, lane, acc[7 + nb]);
+  for (int nb = 0; nb < 5; nb++)
+    write_tile(row, wbase, bbase, kHid, kHid, mb, nb, lane, acc[nb]);
+  if (group) {
+    write_tile(row, kW4, kB4, kHid, kOut, 0, mb, lane, acc[5]);
+    if (mb == 0) write_tile(row, kW4, kB4, kHid, kOut, 0, 4, lane, acc[6]);
+  } else {
+    write_tile(row, kW1, kB1, kIn, kHid, mb, 0, lane, acc[5]);
   }
-  write_tile(row, kW1, kB1, kIn, kHid, wave, 0, lane, acc[12]);
-  for (int d = 32; d >= 1; d >>= 1) lsum += __shfl_xor(lsum, d, 64);
-  if (lane == 0) sloss[wave] = lsum;
+  if (mb == 0) {
+    for (int d = 32; d >= 1; d >>= 1) lsum += __shfl_xor(lsum, d, 64);
+    if (lane == 0) sloss[group] = lsum;
+  }
   __syncthreads();
-  if (threadIdx.x == 0)
-    partial_loss[blockIdx.x] = ((sloss[0] + sloss[1]) + sloss[2]) + sloss[3];
+  if (threadIdx.x == 0) partial_loss[blockIdx.x] = sloss[0] + sloss[1];
 }
 
 // Parameter k's places among the packed operands (the inverse of mlp_pack_kernel's map).
@@ -474,21 +459,25 @@ __device__ __forceinline__ void pack_one(uint16_t* __restrict__ packed, int k, f
   }
 }
 
-constexpr int kAdamThreads = 64;
+constexpr int kAdamParams = 64;  // per workgroup, whose waves take a part of the rows each
+constexpr int kAdamWaves = 4;
 constexpr int kAdamRows = 16;  // rows in flight per lane
 
-// Sums the workgroups' gradient rows in order; optionally writes the gradient and/or
+// Sums the workgroups' gradient rows (kAdamWaves runs of rows, then those sums); optionally writes the gradient and/or
 // applies Adam to the master weights, whose packed operands (all zero where they hold no
 // weight) it rewrites.  The last workgroup sums the partial losses in order.  Bound by the
-// latency of the row loads: a wave per workgroup and 16 rows in flight instead of 256 lanes and
-// the few rows of the compiler's own unrolling, 4.6 us at 64 rows (16.6 us, and 9.9 us for the
+// latency of the row loads, hence four waves and 16 rows in flight each: 5.9 us at 128 rows
+// (16.6 us at 64 rows with 37 workgroups of the compiler's own unrolling, and 9.9 us for the
 // losses and operands as launches of their own).
-__global__ void __launch_bounds__(kAdamThreads) mlp_adam_kernel(
+__global__ void __launch_bounds__(kAdamParams* kAdamWaves) mlp_adam_kernel(
     float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
     uint16_t* __restrict__ packed, const float* __restrict__ partial,
     const float* __restrict__ partial_loss, uint32_t rows, float* __restrict__ grad_out,
     float* __restrict__ loss_out, int update, float lr, float c1, float c2) {
+  __shared__ float sums[kAdamWaves][kAdamParams];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   if (blockIdx.x == gridDim.x - 1) {
+    if (wave != 0) return;
     float s = 0.0f;
     for (uint32_t r0 = 0; r0 < rows; r0 += 64) {
       const uint32_t r = r0 + threadIdx.x;
@@ -500,19 +489,27 @@ __global__ void __launch_bounds__(kAdamThreads) mlp_adam_kernel(
     if (threadIdx.x == 0) *loss_out = s;
     return;
   }
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= (uint32_t)kMlpParams) return;
-  const float* at = partial + k;
+  const uint32_t k = blockIdx.x * kAdamParams + lane;
   float gsum = 0.0f;
-  uint32_t r = 0;
-  for (; r + kAdamRows <= rows; r += kAdamRows, at += (size_t)kAdamRows * kMlpParams) {
-    float x[kAdamRows];
+  if (k < (uint32_t)kMlpParams) {
+    const uint32_t per = (rows + kAdamWaves - 1) / kAdamWaves;
+    uint32_t r = min(wave * per, rows);
+    const uint32_t end = min(r + per, rows);
+    const float* at = partial + (size_t)r * kMlpParams + k;
+    for (; r + kAdamRows <= end; r += kAdamRows, at += (size_t)kAdamRows * kMlpParams) {
+      float x[kAdamRows];
 #pragma unroll
-    for (int q = 0; q < kAdamRows; q++) x[q] = at[(size_t)q * kMlpParams];
+      for (int q = 0; q < kAdamRows; q++) x[q] = at[(size_t)q * kMlpParams];
 #pragma unroll
-    for (int q = 0; q < kAdamRows; q++) gsum += x[q];
+      for (int q = 0; q < kAdamRows; q++) gsum += x[q];
+    }
+    for (; r < end; r++, at += kMlpParams) gsum += *at;
   }
-  for (; r < rows; r++, at += kMlpParams) gsum += *at;
+  sums[wave][lane] = gsum;
+  __syncthreads();
+  if (wave != 0 || k >= (uint32_t)kMlpParams) return;
+#pragma unroll
+  for (int q = 1; q < kAdamWaves; q++) gsum += sums[q][lane];
   if (grad_out) grad_out[k] = gsum;
   if (!update) return;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
@@ -546,7 +543,7 @@ unsigned mlp_grad_rows(size_t count) {
 void mlp_grad(splat_ctx* ctx, const void* packed, const float* params, const float* feats,
               const uint8_t* labels, const float* weights, const uint32_t* order, size_t count,
               float inv_batch, float* partial, float* partial_loss) {
-  launch(ctx, "mlp_grad", mlp_grad_kernel, dim3(mlp_grad_rows(count)), dim3(256), 0,
+  launch(ctx, "mlp_grad", mlp_grad_kernel, dim3(mlp_grad_rows(count)), dim3(kGradThreads), 0,
          (const bf16x8*)packed, params, feats, labels, weights, order, (uint32_t)count,
          inv_batch, partial, partial_loss);
 }
@@ -555,8 +552,8 @@ void mlp_reduce_update(splat_ctx* ctx, float* params, float* m, float* v, void* 
                        const float* partial, const float* partial_loss, unsigned rows,
                        float* grad_out, float* loss_out, bool update, float lr, float c1,
                        float c2) {
-  launch(ctx, "mlp_adam", mlp_adam_kernel, dim3(blocks_for(kMlpParams, kAdamThreads) + 1),
-         dim3(kAdamThreads), 0, params, m, v, (uint16_t*)packed, partial, partial_loss, rows,
+  launch(ctx, "mlp_adam", mlp_adam_kernel, dim3(blocks_for(kMlpParams, kAdamParams) + 1),
+         dim3(kAdamParams * kAdamWaves), 0, params, m, v, (uint16_t*)packed, partial, partial_loss, rows,
          grad_out, loss_out, update ? 1 : 0, lr, c1, c2);
 }
 
