@@ -12,7 +12,7 @@
 // units the lane holds, and the weight operands are packed in the same permuted order.
 //
 // Weight gradients contract over samples, so the error signals and activations of a
-// 32-sample chunk are staged in LDS transposed ([unit][sample]) and multiplied there; a
+// 64-sample chunk are staged in LDS transposed ([unit][sample]) and multiplied there; a
 // constant-one input turns the bias gradients into one more output column.
 //
 // Parameter layout (binary32 master copy): W1[64][12] b1[64] W2[64][64] b2[64] W3[64][64]
@@ -34,11 +34,12 @@ constexpr int kW1 = 0, kB1 = 768, kW2 = 832, kB2 = 4928, kW3 = 4992, kB3 = 9088,
 // layers 4, 3, 2 (4x1, 4x2, 4x2).
 constexpr int kF1 = 0, kF2 = 4, kF3 = 12, kF4 = 20, kT4 = 22, kT3 = 26, kT2 = 34,
               kBlocks = 42;
-constexpr int kChunk = 32;  // samples per workgroup pass of the training kernel
-// bfloat16 values between the LDS rows of two units: 80 bytes, so that the 16 rows which a
+constexpr int kChunk = 64;  // samples per workgroup pass of the training kernel
+constexpr int kGroups = kChunk / 16;  // samples in groups of 16, one per column of a matrix tile
+// bfloat16 values between the LDS rows of two units: 144 bytes, so that the 16 rows which a
 // matrix operand is read from, 16 bytes each, lie in different banks
 constexpr int kRow = kChunk + 8;
-constexpr int kGradThreads = 512;
+constexpr int kGradThreads = 64 * 4 * kGroups;  // a wave per sample group and M-block
 
 __device__ __forceinline__ __bf16 to_bf16(float x) {  // round to nearest, ties to even
   uint32_t u = __float_as_uint(x);
@@ -94,7 +95,7 @@ __device__ __forceinline__ float gelu(float z, const uint64_t* tab, float* dg) {
 }
 
 __device__ __forceinline__ bf16x8 blockop(const bf16x8* __restrict__ packed, int block, int lane) {
-  return packed[block * 64 + lane];
+  return (packed + block * 64)[(uint32_t)lane];  // uniform base, 32-bit lane offset
 }
 
 // B operand (slot kb) from the D values of four M-blocks.
@@ -271,9 +272,10 @@ __device__ __forceinline__ void stage(uint16_t* s, uint2 v, int mb, int lane, in
   at[3 * kRow] = (uint16_t)(v.y >> 16);
 }
 
-// The operand of 16 units over the staged samples.
-__device__ __forceinline__ bf16x8 staged(const uint16_t* s, int mb, int lane) {
-  return *reinterpret_cast<const bf16x8*>(s + (16 * mb + (lane & 15)) * kRow + 8 * (lane >> 4));
+// The operand of 16 units over staged samples 32 kb .. 32 kb + 31.
+__device__ __forceinline__ bf16x8 staged(const uint16_t* s, int mb, int kb, int lane) {
+  return *reinterpret_cast<const bf16x8*>(s + (16 * mb + (lane & 15)) * kRow + 32 * kb +
+                                          8 * (lane >> 4));
 }
 
 // Write a 16x16 tile of weight gradients (row block mb, column block nb; `nin` columns are
@@ -295,16 +297,18 @@ __device__ __forceinline__ void write_tile(float* __restrict__ row, int wbase, i
 // Gradient of the weighted binary cross-entropy over `count` samples (ids order[0..count)
 // or 0..count), scaled by inv_batch.  Each workgroup accumulates its chunks' weight
 // gradients in registers and writes one partial gradient row (kMlpParams floats) plus its
-// partial loss; mlp_adam_kernel sums the rows.
+// partial loss; mlp_adam_kernel sums the rows in workgroup order.
 //
-// Wave w has sample group w % 2 (16 samples) and M-block w / 2 (16 units) of every hidden layer:
-// a layer's values are exchanged through LDS, where the weight gradients find them too (row
-// block w / 2 of layers 3 and 1 on the even waves, of layer 2 on the odd ones, and layer 4's
-// column block w / 2).  Bound by the
-// chain of seven layers, mostly the vector instructions of the activations: a wave has 12 per
-// lane.  A batch of 4096 makes 128 workgroups, 15.2 us; 64 workgroups of four waves with 48
-// activations per lane took 22.5 us, and 31.7 us with two barriers per layer and LDS rows of
-// 128 bytes, all in the same banks.
+// Wave w has sample group w % 4 (16 samples) and M-block w / 4 (16 units) of every hidden layer:
+// a layer's values are exchanged through LDS, where the weight gradients find them too.  Of
+// those, the waves of M-block mb take layers 3 and 2's row block mb (groups 0 and 1 layer 3's
+// columns, 2 and 3 layer 2's), layer 1's (group 1) and layer 4's column block mb (group 3).
+// Every tile is summed over a chunk's 64 samples in one accumulator and over the rows in
+// order.  Bound by the chain of seven layers, mostly the vector instructions of the
+// activations: a wave has 12 per lane, four waves share a SIMD.  A batch of 4096 makes 64
+// workgroups, 20.7 us; workgroups of four waves with 48 activations per lane took 22.5 us, and
+// 31.7 us with two barriers per layer and LDS rows of 128 bytes, all in the same banks.  (128
+// workgroups of 32 samples took 15.2 us, but sum each weight gradient in other parts.)
 __global__ void __launch_bounds__(kGradThreads) mlp_grad_kernel(
     const bf16x8* __restrict__ packed, const float* __restrict__ p,
     const float* __restrict__ feats, const uint8_t* __restrict__ labels,
@@ -314,18 +318,19 @@ __global__ void __launch_bounds__(kGradThreads) mlp_grad_kernel(
   __shared__ __attribute__((aligned(16))) uint16_t sE4[16 * kRow], sE3[64 * kRow],
       sE2[64 * kRow], sE1[64 * kRow], sA3[64 * kRow], sA2[64 * kRow], sA1[64 * kRow],
       sX[16 * kRow];
-  __shared__ uint2 exch[5][2][4][64];  // activations 1 to 3, errors 3 and 2; group, M-block, lane
-  __shared__ float sloss[2];
+  __shared__ uint2 exch[5][kGroups][4][64];  // activations 1 to 3, errors 3 and 2; group, M-block, lane
+  __shared__ float sloss[kGroups];
   __shared__ uint64_t tab[32];
   load_exp_table(tab);
   __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4;
-  const int group = wave & 1, mb = wave >> 1;
-  // four column blocks and the bias of layer 3 (even waves) or 2; layer 1 (even) or layer 4 and
-  // its bias
-  f32x4 acc[7];
+  const int lane = threadIdx.x & 63, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int group = wave % kGroups, mb = wave / kGroups;
+  // columns of layer 3 (groups 0, 1) or 2: blocks 0 to 2 (even groups) or block 3 and the bias;
+  // then layer 1 (group 1) or layer 4 and its bias (group 3)
+  f32x4 acc[4];
 #pragma unroll
-  for (int k = 0; k < 7; k++) acc[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int k = 0; k < 4; k++) acc[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   const __bf16 one = (lane & 15) == 0 ? __builtin_bit_cast(__bf16, (uint16_t)0x3F80)
                                       : __builtin_bit_cast(__bf16, (uint16_t)0);
   const bf16x8 ones = {one, one, one, one, one, one, one, one};  // the constant-one input
@@ -350,23 +355,45 @@ __global__ void __launch_bounds__(kGradThreads) mlp_grad_kernel(
     const float w = valid ? weights[s] : 0.0f;
     const uint32_t y = valid ? labels[s] : 0u;
     const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (mb == 0 && g < 2) {
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const int k = 8 * g + q;
+        const float x = k < kIn ? f[k] : 0.0f;
+        sX[k * kRow + 16 * group + (lane & 15)] = k == kIn ? 0x3F80 : bf16_bits(x);
+      }
+    }
+    // A layer's operands and bias are loaded no earlier than beside the layer before it: all
+    // layers' would not fit the 128 registers of a lane.
+    const bf16x8* at = packed;
+    const float* bias = p;
+    const auto next_layer = [&] {
+      at = reload(at);
+      bias = reload(bias);
+    };
+    next_layer();
     f32x4 d1, d2, d3;
     bf16x8 b0, b1;
-    uint2 v = pack4(gelu4(mfma(blockop(packed, kF1 + mb, lane), feature_operand(f, g),
-                               bias4(p + kB1, mb, g)),
-                          tab, &d1));
+    f32x4 z = mfma(blockop(at, kF1 + mb, lane), feature_operand(f, g), bias4(bias + kB1, mb, g));
+    next_layer();
+    uint2 v = pack4(gelu4(z, tab, &d1));
     stage(sA1, v, mb, lane, group);
     exchange(0, v, &b0, &b1);
-    f32x4 z = mfma(blockop(packed, kF2 + 2 * mb, lane), b0, bias4(p + kB2, mb, g));
-    v = pack4(gelu4(mfma(blockop(packed, kF2 + 2 * mb + 1, lane), b1, z), tab, &d2));
+    z = mfma(blockop(at, kF2 + 2 * mb, lane), b0, bias4(bias + kB2, mb, g));
+    z = mfma(blockop(at, kF2 + 2 * mb + 1, lane), b1, z);
+    next_layer();
+    v = pack4(gelu4(z, tab, &d2));
     stage(sA2, v, mb, lane, group);
     exchange(1, v, &b0, &b1);
-    z = mfma(blockop(packed, kF3 + 2 * mb, lane), b0, bias4(p + kB3, mb, g));
-    v = pack4(gelu4(mfma(blockop(packed, kF3 + 2 * mb + 1, lane), b1, z), tab, &d3));
+    z = mfma(blockop(at, kF3 + 2 * mb, lane), b0, bias4(bias + kB3, mb, g));
+    z = mfma(blockop(at, kF3 + 2 * mb + 1, lane), b1, z);
+    next_layer();
+    v = pack4(gelu4(z, tab, &d3));
     stage(sA3, v, mb, lane, group);
     exchange(2, v, &b0, &b1);
-    z = mfma(blockop(packed, kF4, lane), b0, bias_d(p + kB4, kOut, 0, g));
-    z = mfma(blockop(packed, kF4 + 1, lane), b1, z);
+    z = mfma(blockop(at, kF4, lane), b0, bias_d(bias + kB4, kOut, 0, g));
+    z = mfma(blockop(at, kF4 + 1, lane), b1, z);
+    next_layer();
     // output error (rows 0..2 live in lanes g == 0), on each of the group's waves
     f32x4 e4 = none;
     if (g == 0 && valid) {
@@ -381,57 +408,61 @@ __global__ void __launch_bounds__(kGradThreads) mlp_grad_kernel(
     v = pack4(e4);
     if (mb == 0) stage(sE4, v, 0, lane, group);
     const bf16x8 E = __builtin_bit_cast(bf16x8, make_uint4(v.x, v.y, 0u, 0u));
-    v = pack4(mfma(blockop(packed, kT4 + mb, lane), E, none) * d3);
+    v = pack4(mfma(blockop(at, kT4 + mb, lane), E, none) * d3);
     stage(sE3, v, mb, lane, group);
     exchange(3, v, &b0, &b1);
-    z = mfma(blockop(packed, kT3 + 2 * mb, lane), b0, none);
-    v = pack4(mfma(blockop(packed, kT3 + 2 * mb + 1, lane), b1, z) * d2);
+    z = mfma(blockop(at, kT3 + 2 * mb, lane), b0, none);
+    v = pack4(mfma(blockop(at, kT3 + 2 * mb + 1, lane), b1, z) * d2);
     stage(sE2, v, mb, lane, group);
     exchange(4, v, &b0, &b1);
-    z = mfma(blockop(packed, kT2 + 2 * mb, lane), b0, none);
-    v = pack4(mfma(blockop(packed, kT2 + 2 * mb + 1, lane), b1, z) * d1);
+    z = mfma(blockop(at, kT2 + 2 * mb, lane), b0, none);
+    v = pack4(mfma(blockop(at, kT2 + 2 * mb + 1, lane), b1, z) * d1);
     stage(sE1, v, mb, lane, group);
-    if (mb == 0 && g < 2) {
-#pragma unroll
-      for (int q = 0; q < 8; q++) {
-        const int k = 8 * g + q;
-        const float x = k < kIn ? f[k] : 0.0f;
-        sX[k * kRow + 16 * group + (lane & 15)] = k == kIn ? 0x3F80 : bf16_bits(x);
-      }
-    }
     __syncthreads();
-    const uint16_t *se = group ? sE2 : sE3, *sa = group ? sA1 : sA2;
-    const bf16x8 e = staged(se, mb, lane);
+    const uint16_t *se = group < 2 ? sE3 : sE2, *sa = group < 2 ? sA2 : sA1;
 #pragma unroll
-    for (int nb = 0; nb < 4; nb++) acc[nb] = mfma(e, staged(sa, nb, lane), acc[nb]);
-    acc[4] = mfma(e, ones, acc[4]);
-    if (group) {
-      const bf16x8 e4b = staged(sE4, 0, lane);
-      acc[5] = mfma(e4b, staged(sA3, mb, lane), acc[5]);
-      acc[6] = mfma(e4b, ones, acc[6]);
-    } else {
-      acc[5] = mfma(staged(sE1, mb, lane), staged(sX, 0, lane), acc[5]);
+    for (int kb = 0; kb < kChunk / 32; kb++) {
+      const bf16x8 e = staged(se, mb, kb, lane);
+      if (group % 2 == 0) {
+#pragma unroll
+        for (int nb = 0; nb < 3; nb++) acc[nb] = mfma(e, staged(sa, nb, kb, lane), acc[nb]);
+      } else {
+        acc[0] = mfma(e, staged(sa, 3, kb, lane), acc[0]);
+        acc[1] = mfma(e, ones, acc[1]);
+      }
+      if (group == 1) {
+        acc[2] = mfma(staged(sE1, mb, kb, lane), staged(sX, 0, kb, lane), acc[2]);
+      } else if (group == 3) {
+        const bf16x8 e4b = staged(sE4, 0, kb, lane);
+        acc[2] = mfma(e4b, staged(sA3, mb, kb, lane), acc[2]);
+        acc[3] = mfma(e4b, ones, acc[3]);
+      }
     }
     __syncthreads();
   }
   // write this workgroup's gradient row
   float* row = partial + (size_t)blockIdx.x * kMlpParams;
-  const int wbase = group ? kW2 : kW3, bbase = group ? kB2 : kB3;
+  const int wbase = group < 2 ? kW3 : kW2, bbase = group < 2 ? kB3 : kB2;
+  if (group % 2 == 0) {
 #pragma unroll
-  for (int nb = 0; nb < 5; nb++)
-    write_tile(row, wbase, bbase, kHid, kHid, mb, nb, lane, acc[nb]);
-  if (group) {
-    write_tile(row, kW4, kB4, kHid, kOut, 0, mb, lane, acc[5]);
-    if (mb == 0) write_tile(row, kW4, kB4, kHid, kOut, 0, 4, lane, acc[6]);
+    for (int nb = 0; nb < 3; nb++) write_tile(row, wbase, bbase, kHid, kHid, mb, nb, lane, acc[nb]);
   } else {
-    write_tile(row, kW1, kB1, kIn, kHid, mb, 0, lane, acc[5]);
+    write_tile(row, wbase, bbase, kHid, kHid, mb, 3, lane, acc[0]);
+    write_tile(row, wbase, bbase, kHid, kHid, mb, 4, lane, acc[1]);
+  }
+  if (group == 1) {
+    write_tile(row, kW1, kB1, kIn, kHid, mb, 0, lane, acc[2]);
+  } else if (group == 3) {
+    write_tile(row, kW4, kB4, kHid, kOut, 0, mb, lane, acc[2]);
+    if (mb == 0) write_tile(row, kW4, kB4, kHid, kOut, 0, 4, lane, acc[3]);
   }
   if (mb == 0) {
     for (int d = 32; d >= 1; d >>= 1) lsum += __shfl_xor(lsum, d, 64);
     if (lane == 0) sloss[group] = lsum;
   }
   __syncthreads();
-  if (threadIdx.x == 0) partial_loss[blockIdx.x] = sloss[0] + sloss[1];
+  if (threadIdx.x == 0)
+    partial_loss[blockIdx.x] = ((sloss[0] + sloss[1]) + sloss[2]) + sloss[3];
 }
 
 // Parameter k's places among the packed operands (the inverse of mlp_pack_kernel's map).
@@ -459,25 +490,21 @@ __device__ __forceinline__ void pack_one(uint16_t* __restrict__ packed, int k, f
   }
 }
 
-constexpr int kAdamParams = 64;  // per workgroup, whose waves take a part of the rows each
-constexpr int kAdamWaves = 4;
+constexpr int kAdamThreads = 64;
 constexpr int kAdamRows = 16;  // rows in flight per lane
 
-// Sums the workgroups' gradient rows (kAdamWaves runs of rows, then those sums); optionally writes the gradient and/or
+// Sums the workgroups' gradient rows in order; optionally writes the gradient and/or
 // applies Adam to the master weights, whose packed operands (all zero where they hold no
 // weight) it rewrites.  The last workgroup sums the partial losses in order.  Bound by the
-// latency of the row loads, hence four waves and 16 rows in flight each: 5.9 us at 128 rows
-// (16.6 us at 64 rows with 37 workgroups of the compiler's own unrolling, and 9.9 us for the
+// latency of the row loads: a wave per workgroup and 16 rows in flight instead of 256 lanes and
+// the few rows of the compiler's own unrolling, 5.2 us at 64 rows (16.6 us, and 9.9 us for the
 // losses and operands as launches of their own).
-__global__ void __launch_bounds__(kAdamParams* kAdamWaves) mlp_adam_kernel(
+__global__ void __launch_bounds__(kAdamThreads) mlp_adam_kernel(
     float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
     uint16_t* __restrict__ packed, const float* __restrict__ partial,
     const float* __restrict__ partial_loss, uint32_t rows, float* __restrict__ grad_out,
     float* __restrict__ loss_out, int update, float lr, float c1, float c2) {
-  __shared__ float sums[kAdamWaves][kAdamParams];
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
   if (blockIdx.x == gridDim.x - 1) {
-    if (wave != 0) return;
     float s = 0.0f;
     for (uint32_t r0 = 0; r0 < rows; r0 += 64) {
       const uint32_t r = r0 + threadIdx.x;
@@ -489,27 +516,19 @@ __global__ void __launch_bounds__(kAdamParams* kAdamWaves) mlp_adam_kernel(
     if (threadIdx.x == 0) *loss_out = s;
     return;
   }
-  const uint32_t k = blockIdx.x * kAdamParams + lane;
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= (uint32_t)kMlpParams) return;
+  const float* at = partial + k;
   float gsum = 0.0f;
-  if (k < (uint32_t)kMlpParams) {
-    const uint32_t per = (rows + kAdamWaves - 1) / kAdamWaves;
-    uint32_t r = min(wave * per, rows);
-    const uint32_t end = min(r + per, rows);
-    const float* at = partial + (size_t)r * kMlpParams + k;
-    for (; r + kAdamRows <= end; r += kAdamRows, at += (size_t)kAdamRows * kMlpParams) {
-      float x[kAdamRows];
+  uint32_t r = 0;
+  for (; r + kAdamRows <= rows; r += kAdamRows, at += (size_t)kAdamRows * kMlpParams) {
+    float x[kAdamRows];
 #pragma unroll
-      for (int q = 0; q < kAdamRows; q++) x[q] = at[(size_t)q * kMlpParams];
+    for (int q = 0; q < kAdamRows; q++) x[q] = at[(size_t)q * kMlpParams];
 #pragma unroll
-      for (int q = 0; q < kAdamRows; q++) gsum += x[q];
-    }
-    for (; r < end; r++, at += kMlpParams) gsum += *at;
+    for (int q = 0; q < kAdamRows; q++) gsum += x[q];
   }
-  sums[wave][lane] = gsum;
-  __syncthreads();
-  if (wave != 0 || k >= (uint32_t)kMlpParams) return;
-#pragma unroll
-  for (int q = 1; q < kAdamWaves; q++) gsum += sums[q][lane];
+  for (; r < rows; r++, at += kMlpParams) gsum += *at;
   if (grad_out) grad_out[k] = gsum;
   if (!update) return;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
@@ -552,8 +571,8 @@ void mlp_reduce_update(splat_ctx* ctx, float* params, float* m, float* v, void* 
                        const float* partial, const float* partial_loss, unsigned rows,
                        float* grad_out, float* loss_out, bool update, float lr, float c1,
                        float c2) {
-  launch(ctx, "mlp_adam", mlp_adam_kernel, dim3(blocks_for(kMlpParams, kAdamParams) + 1),
-         dim3(kAdamParams * kAdamWaves), 0, params, m, v, (uint16_t*)packed, partial, partial_loss, rows,
+  launch(ctx, "mlp_adam", mlp_adam_kernel, dim3(blocks_for(kMlpParams, kAdamThreads) + 1),
+         dim3(kAdamThreads), 0, params, m, v, (uint16_t*)packed, partial, partial_loss, rows,
          grad_out, loss_out, update ? 1 : 0, lr, c1, c2);
 }
 

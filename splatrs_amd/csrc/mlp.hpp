@@ -21,7 +21,7 @@ unsigned mlp_grad_rows(size_t count);
 void mlp_grad(splat_ctx* ctx, const void* packed, const float* params, const float* feats,
               const uint8_t* labels, const float* weights, const uint32_t* order, size_t count,
               float inv_batch, float* partial, float* partial_loss);
-// Sums of the partial rows -> grad_out (optional) and of the partial losses ->
+// Sums of the partial rows (in row order) -> grad_out (optional) and of the partial losses ->
 // loss_out; when `update`, Adam on the master weights and their packed operands, which mlp_pack
 // has written before.
 void mlp_reduce_update(splat_ctx* ctx, float* params, float* m, float* v, void* packed,
