@@ -15,7 +15,8 @@
 //      512 entries by one wave each (a bitonic network in registers, lanes exchanging
 //      by DPP and the gfx950 row swaps), larger ones by a workgroup of eight waves that sort
 //      runs and rank every entry in the other runs (in LDS up to 4096 entries; beyond,
-//      chunks of 4096 are ranked through global memory).  This equals the reference's (key, entry) order.
+//      chunks of 4096 are merged pair by pair through global memory).  This equals the
+//      reference's (key, entry) order.
 #include "internal.hpp"
 
 namespace splat {
@@ -425,6 +426,14 @@ __global__ void __launch_bounds__(256) sort_tiles_kernel(uint32_t num_tiles,
     wave_sort_tile<8>(lane, tile, s, n, bucket, sorted_entry, sorted_gauss, keys_out);
 }
 
+// threadIdx.x, but nothing computed from it is known to be the same as elsewhere: keeps what the
+// sorts of the other sizes index with from being held in registers across a sort.
+__device__ __forceinline__ uint32_t own_thread() {
+  uint32_t t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 // Sorts the n <= 64 K kRunWaves records at bucket[s ..]: each wave sorts a run of 64 K in
 // registers, the runs' keys go to LDS, and an entry's place is its place in its own run plus
 // the number of smaller keys in every other run (binary searches of 8 entries' worth of
@@ -436,7 +445,7 @@ template <int K, class Put>
 __device__ __forceinline__ void run_sort(uint32_t s, uint32_t n, const uint4* bucket,
                                          uint64_t* sh, Put&& put) {
   constexpr uint32_t L = 64 * K;  // a run
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint32_t tid = own_thread(), lane = tid & 63u, wave = tid >> 6;
   uint64_t key[K];
   uint32_t gid[K], place[K];
 #pragma unroll
@@ -488,18 +497,202 @@ __device__ __forceinline__ void run_sort(uint32_t s, uint32_t n, const uint4* bu
     if (key[k] != ~0ull) put(place[k], key[k], gid[k]);
 }
 
+// ---- tiles beyond kRunCap entries ---------------------------------------------------
+// Such a tile's 16-byte records make room for its 8-byte keys twice, as `from` and `to`: chunks
+// of kRunCap records are sorted and their keys stored from the front on (behind records that
+// are read by then); the chunks are merged pair by pair, then pairs of those, and so on.  A key
+// names its entry, which has the Gaussian.  n log n; a bitonic network (in LDS by 1024 lanes up
+// to 16384 entries, in global memory beyond) is n log^2 n, and ranking every key in every other
+// chunk n^2.  One tile of n entries, in us, this / network / ranks: 5000 38 / 65 / 72, 8000
+// 44 / 83 / 106, 16000 98 / 166 / 313, 64000 484 / 2160 / 3730, 256000 2320 / 10600 / 99000,
+// 1000000 11800 / 66700 / 1660000; a hundred tiles of 16000 113 / 183 / 459.  (With a search
+// per key instead of a merge per lane: 193 at 16000, bound by the LDS reads.)
+
+__device__ __forceinline__ uint64_t key_of(uint2 k) { return ((uint64_t)k.y << 32) | k.x; }
+__device__ __forceinline__ uint2 key_words(uint64_t k) {
+  return make_uint2((uint32_t)k, (uint32_t)(k >> 32));
+}
+
+constexpr uint32_t kRunThreads = 64 * kRunWaves;
+constexpr uint32_t kPerLane = kRunCap / kRunThreads;  // keys per lane of a chunk
+
+// A chunk's keys in LDS lie one word pair further apart every kPerLane keys: the lanes' own
+// kPerLane consecutive keys start in different banks.
+constexpr uint32_t kChunkWords = kRunCap + kRunCap / kPerLane;
+__device__ __forceinline__ uint32_t padded(uint32_t i) { return i + i / kPerLane; }
+
+// Keys d .. d + kPerLane - 1 of the merge of the sorted keys a .. a + na and b .. b + nb of the
+// chunk in `sh`, all ones past the end (d <= na + nb; keys are distinct).
+__device__ __forceinline__ void merge_lane(const uint64_t* sh, uint32_t a, uint32_t na, uint32_t b,
+                                           uint32_t nb, uint32_t d, uint64_t (&out)[kPerLane]) {
+  uint32_t lo = d > nb ? d - nb : 0u, hi = min(d, na);  // how many of the first d are of a
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) / 2;
+    const bool before = sh[padded(a + mid)] < sh[padded(b + d - 1 - mid)];
+    lo = before ? mid + 1 : lo;
+    hi = before ? hi : mid;
+  }
+  const uint32_t aend = a + na, bend = b + nb;
+  a += lo;
+  b += d - lo;
+  uint64_t x = a < aend ? sh[padded(a)] : ~0ull, y = b < bend ? sh[padded(b)] : ~0ull;
+#pragma unroll
+  for (uint32_t k = 0; k < kPerLane; k++) {
+    const bool take_a = x < y;
+    out[k] = take_a ? x : y;
+    a += take_a ? 1u : 0u;
+    b += take_a ? 0u : 1u;
+    const bool more = take_a ? a < aend : b < bend;
+    const uint64_t v = more ? sh[padded(take_a ? a : b)] : ~0ull;
+    x = take_a ? v : x;
+    y = take_a ? y : v;
+  }
+}
+
+// A chunk's runs of W sorted keys in `sh` (n keys in all) to runs of 2 W, and so on until one is
+// left.  Synchronises before and after each round.
+template <uint32_t W>
+__device__ __forceinline__ void merge_runs(uint64_t* sh, uint32_t n) {
+  const uint32_t t0 = own_thread() * kPerLane, base = t0 / (2 * W) * (2 * W);
+  const uint32_t na = base < n ? min(W, n - base) : 0u;
+  const uint32_t nb = base + W < n ? min(W, n - base - W) : 0u;
+  uint64_t out[kPerLane];
+  __syncthreads();
+  if (t0 < n) merge_lane(sh, base, na, base + W, nb, t0 - base, out);
+  __syncthreads();
+  if (t0 < n) {
+#pragma unroll
+    for (uint32_t k = 0; k < kPerLane; k++) sh[padded(t0 + k)] = out[k];
+  }
+  if constexpr (W * 2 < kRunCap)
+    merge_runs<W * 2>(sh, n);
+  else
+    __syncthreads();
+}
+
+// The keys of the n <= kRunCap records at bucket[s ..], sorted, to out[0 .. n).  All records are
+// read before the first key is written.  `sh` may be reused after a barrier.
+__device__ __forceinline__ void sort_chunk(uint32_t s, uint32_t n, const uint4* bucket,
+                                           uint64_t* sh, uint2* out) {
+  constexpr uint32_t L = 64 * kPerLane;
+  const uint32_t tid = own_thread(), lane = tid & 63u, wave = tid >> 6;
+  uint64_t key[kPerLane];
+  uint32_t none[kPerLane] = {};
+#pragma unroll
+  for (uint32_t k = 0; k < kPerLane; k++) {
+    const uint32_t p = wave * L + k * 64u + lane;
+    const uint4 r = p < n ? bucket[s + p] : make_uint4(~0u, ~0u, 0u, 0u);
+    key[k] = ((uint64_t)r.y << 32) | r.x;
+  }
+  wave_sort_stages<(int)kPerLane, 2, 1>(key, none, lane);
+#pragma unroll
+  for (uint32_t k = 0; k < kPerLane; k++) sh[padded(tid * kPerLane + k)] = key[k];
+  merge_runs<L>(sh, n);
+  for (uint32_t t = tid; t < n; t += kRunThreads) out[t] = key_words(sh[padded(t)]);
+}
+
+// Merges the sorted chunks of kRunCap keys at from[0 .. n) (n > kRunCap; `to` holds n keys too);
+// emit(place, key, Gaussian) takes the entries in the last round.  Every round writes segments of kRunCap keys
+// one after the other: the two runs' parts of a segment (the split of each is found beforehand,
+// by a wave per segment) are staged in LDS and merged there.  Call from every lane.
+constexpr uint32_t kMergeSegments = 512;  // splits held at a time
+template <class Emit>
+__device__ __forceinline__ void merge_chunks(uint2* from, uint2* to, uint32_t n, uint64_t* sh,
+                                             uint32_t* split,
+                                             const uint32_t* __restrict__ entry_gaussian,
+                                             Emit&& emit) {
+  const uint32_t lane = own_thread() & 63u, wave = threadIdx.x >> 6;
+  const uint32_t segments = (n + kRunCap - 1) / kRunCap;
+  for (uint64_t run = kRunCap; run < n; run *= 2) {
+    const bool last = 2 * run >= n;
+    // the pair of runs that segment j is of: its first key, the lengths of its two runs
+    const auto pair_of = [&](uint32_t j, uint32_t* base, uint32_t* la, uint32_t* lb) {
+      *base = (uint32_t)((uint64_t)j * kRunCap & ~(2 * run - 1));
+      *la = (uint32_t)min(run, (uint64_t)(n - *base));
+      *lb = (uint32_t)min(run, (uint64_t)(n - *base - *la));
+    };
+    for (uint32_t j0 = 0; j0 < segments; j0 += kMergeSegments) {
+      const uint32_t held = min(kMergeSegments, segments - j0);
+      // the keys of the first run before each segment, and before the one after the last held
+      for (uint32_t q = wave; q <= held && j0 + q < segments; q += kRunWaves) {
+        uint32_t base, la, lb;
+        pair_of(j0 + q, &base, &la, &lb);
+        const uint2 *a = from + base, *b = a + la;
+        const uint32_t d = (j0 + q) * kRunCap - base;
+        uint32_t lo = d > lb ? d - lb : 0u, hi = min(d, la);  // 64 probes at a time
+        while (lo < hi) {
+          const uint32_t stride = (hi - lo + 63) / 64, p = lo + lane * stride;
+          const bool before = p < hi && key_of(a[p]) < key_of(b[d - 1 - p]);
+          const uint32_t c = (uint32_t)__popcll(__ballot(before));
+          hi = c == 0 ? lo : min(lo + c * stride, hi);
+          lo = c == 0 ? lo : lo + (c - 1) * stride + 1;
+        }
+        if (lane == 0) split[q] = lo;
+      }
+      __syncthreads();
+      for (uint32_t q = 0; q < held; q++) {
+        uint32_t base, la, lb;
+        pair_of(j0 + q, &base, &la, &lb);
+        const uint32_t first = (j0 + q) * kRunCap, d0 = first - base;
+        const uint32_t len = min(kRunCap, la + lb - d0);
+        const uint32_t i0 = split[q], i1 = d0 + len == la + lb ? la : split[q + 1];
+        const uint32_t na = i1 - i0;
+        const uint2 *a = from + base + i0, *b = from + base + la + (d0 - i0);
+        const uint32_t tid = own_thread();
+        uint64_t key[kPerLane];
+#pragma unroll
+        for (uint32_t k = 0; k < kPerLane; k++) {  // no branch between the loads
+          const uint32_t t = min(k * kRunThreads + tid, len - 1);
+          key[k] = key_of(*(t < na ? a + t : b + (t - na)));
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kPerLane; k++) sh[padded(k * kRunThreads + tid)] = key[k];
+        __syncthreads();
+        if (tid * kPerLane < len) merge_lane(sh, 0, na, na, len - na, tid * kPerLane, key);
+        __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < kPerLane; k++) sh[padded(tid * kPerLane + k)] = key[k];
+        __syncthreads();
+        uint32_t gid[kPerLane];
+#pragma unroll
+        for (uint32_t k = 0; k < kPerLane; k++)
+          key[k] = sh[padded(min(k * kRunThreads + tid, len - 1))];
+        if (last) {
+#pragma unroll
+          for (uint32_t k = 0; k < kPerLane; k++) gid[k] = entry_gaussian[(uint32_t)key[k]];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kPerLane; k++) {
+          const uint32_t t = k * kRunThreads + tid;
+          if (t >= len) continue;
+          if (last)
+            emit(first + t, key[k], gid[k]);
+          else
+            to[first + t] = key_words(key[k]);
+        }
+        __syncthreads();  // sh is free; after the last segment, split too, and `to` is written
+      }
+    }
+    uint2* const t = from;
+    from = to;
+    to = t;
+  }
+}
+
 // The queued tiles (more than kWaveCap entries), one workgroup each; the grid strides over the
 // queue.  Bound by the latency of the networks and searches of the largest tiles.  At 300k
 // Gaussians, 1297x840 (1066 such tiles, 335 beyond 1024 entries, up to 3023), this took
-// 39 us where one wave per tile up to 1024 entries and a bitonic sort in LDS by 1024 lanes
+// 33 us (39 us with 21 registers spilled, see own_thread) where one wave per tile up to 1024 entries and a bitonic sort in LDS by 1024 lanes
 // beyond took 28 + 56 us; with a handful of tiles of 500-1000 entries 7 us
 // against 22 + 4, with none 6 us against 5 + 5.
 __global__ void __launch_bounds__(64 * kRunWaves, 4) sort_queue_kernel(
-    const uint32_t* __restrict__ tile_start, uint4* bucket, uint32_t* __restrict__ sorted_entry,
+    const uint32_t* __restrict__ tile_start, uint4* bucket,
+    const uint32_t* __restrict__ entry_gaussian, uint32_t* __restrict__ sorted_entry,
     uint32_t* __restrict__ sorted_gauss, uint64_t* __restrict__ keys_out,
     uint32_t num_tiles, const uint32_t* __restrict__ queue,
     const uint32_t* __restrict__ counts) {
-  __shared__ uint64_t sh[kRunCap];
+  __shared__ uint64_t sh[kChunkWords];
+  __shared__ uint32_t split[kMergeSegments + 1];
   const uint32_t first = counts[0], count = first + counts[2];
   for (uint32_t q = blockIdx.x; q < count; q += gridDim.x) {
     const uint32_t tile = queue[q < first ? q : num_tiles - 1 - (q - first)];
@@ -516,36 +709,12 @@ __global__ void __launch_bounds__(64 * kRunWaves, 4) sort_queue_kernel(
     } else if (n <= kRunCap) {
       run_sort<8>(s, n, bucket, sh, emit);
     } else {
-      // chunks sorted in place, then every entry ranked in the other chunks
+      uint2* const keys = reinterpret_cast<uint2*>(bucket + s);
       for (uint32_t c = 0; c < n; c += kRunCap) {
-        run_sort<8>(s + c, min(kRunCap, n - c), bucket, sh,
-                    [&](uint32_t place, uint64_t key, uint32_t gid) {
-                      bucket[s + c + place] =
-                          make_uint4((uint32_t)key, (uint32_t)(key >> 32), gid, 0u);
-                    });
+        sort_chunk(s + c, min(kRunCap, n - c), bucket, sh, keys + c);
         __syncthreads();
       }
-      const auto key_at = [&](uint32_t i) {
-        const uint2 k = *reinterpret_cast<const uint2*>(&bucket[s + i]);
-        return ((uint64_t)k.y << 32) | k.x;
-      };
-      for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
-        const uint4 r = bucket[s + i];
-        const uint64_t key = ((uint64_t)r.y << 32) | r.x;
-        uint32_t place = i % kRunCap;
-        for (uint32_t c = 0; c < n; c += kRunCap) {
-          if (c == i / kRunCap * kRunCap) continue;
-          uint32_t lo = c, len = min(kRunCap, n - c);  // first entry of the chunk not below key
-          while (len > 0) {
-            const uint32_t half = len / 2;
-            const bool below = key_at(lo + half) < key;
-            lo = below ? lo + half + 1 : lo;
-            len = below ? len - half - 1 : half;
-          }
-          place += lo - c;
-        }
-        emit(place, key, r.z);
-      }
+      merge_chunks(keys, keys + n, n, sh, split, entry_gaussian, emit);
     }
     __syncthreads();  // sh is free
   }
@@ -886,8 +1055,8 @@ void sort_tiles(splat_ctx* ctx, const BinBuffers& bb, size_t T, uint64_t* keys_o
          bb.sorted_entry, bb.sorted_gauss, keys_out, queue, counts);
   // two workgroups at a time per compute unit (16 waves of 128 VGPRs), two more in turn
   launch(ctx, "bin_sort_queue", sort_queue_kernel, dim3((unsigned)std::min<size_t>(T, 1024)),
-         dim3(64 * kRunWaves), 0, (const uint32_t*)bb.tile_start, bb.bucket, bb.sorted_entry,
-         bb.sorted_gauss, keys_out, (uint32_t)T, (const uint32_t*)queue, (const uint32_t*)counts);
+         dim3(64 * kRunWaves), 0, (const uint32_t*)bb.tile_start, bb.bucket,
+         (const uint32_t*)bb.entry_gaussian, bb.sorted_entry, bb.sorted_gauss, keys_out, (uint32_t)T, (const uint32_t*)queue, (const uint32_t*)counts);
 }
 
 }  // namespace
