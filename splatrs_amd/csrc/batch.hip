@@ -523,9 +523,7 @@ int splat_batch_tune(splat_batch* b, const uint32_t* views, uint32_t nviews,
 int splat_batch_set_shapes(splat_batch* b, const splat_tune_result* shapes) {
   return bguard(b, [&] {
     SPLAT_REQUIRE(shapes, "null argument");
-    auto ok_f = [](int v) { return v == 32 || v == 64 || v == 128 || v == 256; };
-    SPLAT_REQUIRE(ok_f(shapes->fwd_batch) && (shapes->bwd_batch == 16 || shapes->bwd_batch == 32),
-                  "unsupported batch shape");
+    SPLAT_REQUIRE(supported_batches(*shapes), "unsupported batch shape");
     b->fwd.fwd_batch = shapes->fwd_batch;
     b->fwd.persistent = shapes->fwd_persistent != 0;
     b->fwd.per_cu = (unsigned)std::max(1, shapes->fwd_per_cu);

@@ -552,13 +552,14 @@ int radix_sort_pairs(splat_ctx* ctx, uint32_t* k0, uint32_t* v0, uint32_t* k1, u
 
 // raster.hip
 // Launch shape of the compositing kernels (results do not depend on it): entries per LDS
-// batch of the forward (32, 64, 128, 256) and of the tree-reduced backward (16, 32),
+// batch of the forward (32, 64, 128, 256) and of the tree-reduced backward (16, 32), or 0 for
+// the default (64 and 32, and for a launch of one view with few tiles kernels made for that),
 // whether a fixed grid of per_cu workgroups per compute unit takes tiles from a counter,
 // and whether each 16-lane row of a backward wave walks its own list of entries (rows)
 // or the wave walks the entries that reach any of its rows.
 struct RasterVariant {
-  int fwd_batch = 64;
-  int bwd_batch = 32;
+  int fwd_batch = 0;
+  int bwd_batch = 0;
   bool persistent = false;
   unsigned per_cu = 4;
   bool rows = true;
@@ -599,6 +600,8 @@ RasterTune tune_raster(splat_ctx* ctx, const ProjBuffers& pb, const BinBuffers& 
                        float* final_t, uint32_t* n_contrib, const float* dimage, bool ordered,
                        float* slots, bool need_abs, const BatchDev* bd, uint32_t* counter);
 void fill_tune_result(const RasterTune& t, splat_tune_result* out);
+// Whether the batch sizes of `shapes` are ones a RasterVariant may have.
+bool supported_batches(const splat_tune_result& shapes);
 
 // dataset.hip: image::imageops::resize(.., Lanczos3) of a device RGB8 image into dst
 // (out_w x out_h), as dataset::load downscales views; synchronises.

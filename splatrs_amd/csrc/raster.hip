@@ -18,7 +18,7 @@
 namespace splat {
 namespace {
 
-// Non-persistent launches of one view with few tiles: each wave's own latency bounds them,
+// Launches of one view with few tiles in the default shape: each wave's own latency bounds them,
 // and registers and LDS are free.  The FEW kernels evaluate a step's pair beside the previous
 // step's state update, without a branch, and take larger batches (fewer barriers).  Forward, in
 // us, FEW with 256-entry batches against 64-entry ones: 256 tiles 39 / 53, 1271 tiles 50 / 57,
@@ -1139,6 +1139,15 @@ __global__ void __launch_bounds__(64) reduce_slots_kernel(const uint32_t* __rest
 
 namespace {
 
+// Whether a launch of one view of T tiles, one workgroup each, takes the FEW kernel: only the
+// default shape does, every other runs as given.
+bool few_fwd(const RasterVariant& rv, unsigned T) {
+  return rv.fwd_batch == 0 && !rv.persistent && T <= kFewTilesFwd;
+}
+bool few_bwd(const RasterVariant& rv, unsigned T) {
+  return rv.bwd_batch == 0 && !rv.persistent && rv.rows && T <= kFewTilesBwd;
+}
+
 // Workgroups of a persistent launch: `per_cu` per compute unit.
 unsigned persistent_grid(splat_ctx* ctx, unsigned per_cu, unsigned tiles) {
   int cus = 0;
@@ -1146,44 +1155,27 @@ unsigned persistent_grid(splat_ctx* ctx, unsigned per_cu, unsigned tiles) {
   return std::max(1u, std::min<unsigned>(tiles, (unsigned)cus * std::max(per_cu, 1u)));
 }
 
-template <int B, bool BATCH, bool PERSIST>
+template <int B, bool BATCH, bool PERSIST, bool FEW = false>
 void fwd_go(splat_ctx* ctx, const ProjBuffers& pb, const BinBuffers& bb, unsigned T,
             uint32_t width, uint32_t height, const float bg[3], float* image, float* final_t,
             uint32_t* n_contrib, const BatchDev& bd, uint32_t* counter, unsigned per_cu) {
-  if constexpr (!BATCH && !PERSIST) {
-    if (T <= kFewTilesFwd)
-      return launch(ctx, "raster_fwd", raster_fwd_kernel<256, false, false, false, true>, dim3(T),
-                    dim3(256), 0, (const float4*)pb.rec, (const uint32_t*)bb.tile_start,
-                    (const uint32_t*)bb.tile_order, (const uint32_t*)bb.sorted_gauss, T,
-                    bb.tiles_x, width, height, bg[0], bg[1], bg[2], image, final_t, n_contrib, bd,
-                    counter, (unsigned long long*)nullptr);
-  }
   if (PERSIST) fill_u32(ctx, counter, kXcds, 0u);
   const unsigned grid = PERSIST ? persistent_grid(ctx, per_cu, T) : T;
-  launch(ctx, "raster_fwd", raster_fwd_kernel<B, BATCH, PERSIST>, dim3(grid), dim3(256), 0,
+  launch(ctx, "raster_fwd", raster_fwd_kernel<B, BATCH, PERSIST, false, FEW>, dim3(grid),
+         dim3(256), 0,
          (const float4*)pb.rec, (const uint32_t*)bb.tile_start, (const uint32_t*)bb.tile_order,
          (const uint32_t*)bb.sorted_gauss, T, bb.tiles_x, width, height, bg[0], bg[1], bg[2],
          image, final_t, n_contrib, bd, counter, (unsigned long long*)nullptr);
 }
 
-template <bool ABS, int BF, bool BATCH, bool PERSIST, bool ROWS>
+template <bool ABS, int BF, bool BATCH, bool PERSIST, bool ROWS, bool FEW = false>
 void bwd_go(splat_ctx* ctx, const ProjBuffers& pb, const BinBuffers& bb, unsigned T,
             uint32_t width, uint32_t height, const float bg[3], const float* final_t,
             const uint32_t* n_contrib, const float* dimage, float* slots, const BatchDev& bd,
             uint32_t* counter, unsigned per_cu) {
-  if constexpr (!BATCH && !PERSIST) {
-    if (T <= kFewTilesBwd)
-      return launch(ctx, "raster_bwd",
-                    raster_bwd_kernel<ABS, 64, false, false, true, false, true>, dim3(T), dim3(256),
-                    0, (const float4*)pb.rec, (const uint32_t*)bb.tile_start,
-                    (const uint32_t*)bb.tile_order, (const uint32_t*)bb.sorted_gauss,
-                    (const uint32_t*)bb.sorted_entry, T, bb.tiles_x, width, height, bg[0], bg[1],
-                    bg[2], final_t, n_contrib, dimage, slots, bd, counter,
-                    (unsigned long long*)nullptr);
-  }
   if (PERSIST) fill_u32(ctx, counter, kXcds, 0u);
   const unsigned grid = PERSIST ? persistent_grid(ctx, per_cu, T) : T;
-  launch(ctx, "raster_bwd", raster_bwd_kernel<ABS, BF, BATCH, PERSIST, ROWS>, dim3(grid),
+  launch(ctx, "raster_bwd", raster_bwd_kernel<ABS, BF, BATCH, PERSIST, ROWS, false, FEW>, dim3(grid),
          dim3(256), 0, (const float4*)pb.rec, (const uint32_t*)bb.tile_start,
          (const uint32_t*)bb.tile_order, (const uint32_t*)bb.sorted_gauss,
          (const uint32_t*)bb.sorted_entry, T, bb.tiles_x, width,
@@ -1216,6 +1208,11 @@ void fwd_pick(splat_ctx* ctx, const RasterVariant& rv, const ProjBuffers& pb,
               const BinBuffers& bb, unsigned T, uint32_t width, uint32_t height,
               const float bg[3], float* image, float* final_t, uint32_t* n_contrib,
               const BatchDev& bd, uint32_t* counter) {
+  if constexpr (!BATCH && !PERSIST) {
+    if (few_fwd(rv, T))
+      return fwd_go<256, false, false, true>(ctx, pb, bb, T, width, height, bg, image, final_t,
+                                             n_contrib, bd, counter, rv.per_cu);
+  }
   switch (rv.fwd_batch) {
     case 32:
       return fwd_go<32, BATCH, PERSIST>(ctx, pb, bb, T, width, height, bg, image, final_t,
@@ -1239,6 +1236,16 @@ void bwd_rows_pick(splat_ctx* ctx, const RasterVariant& rv, const ProjBuffers& p
                    const float* dimage, float* slots, bool need_abs, const BatchDev& bd,
                    uint32_t* counter) {
   const unsigned pc = rv.per_cu;
+  if constexpr (!BATCH && !PERSIST && ROWS) {
+    if (few_bwd(rv, T)) {
+      if (need_abs)
+        return bwd_go<true, 64, false, false, true, true>(ctx, pb, bb, T, width, height, bg,
+                                                          final_t, n_contrib, dimage, slots, bd,
+                                                          counter, pc);
+      return bwd_go<false, 64, false, false, true, true>(ctx, pb, bb, T, width, height, bg, final_t,
+                                                         n_contrib, dimage, slots, bd, counter, pc);
+    }
+  }
   if (rv.bwd_batch == 16) {
     if (need_abs)
       return bwd_go<true, 16, BATCH, PERSIST, ROWS>(ctx, pb, bb, T, width, height, bg, final_t,
@@ -1371,10 +1378,15 @@ RasterTune tune_raster(splat_ctx* ctx, const ProjBuffers& pb, const BinBuffers& 
       }
       return best;
     };
-    const RasterVariant def;
+    // the default shape is a candidate of its own where it is not the 64 / 32 entries it means
+    // on images with more tiles
+    const unsigned T = bb.tiles_x * bb.tiles_y;
+    const int def_fwd = !bd && few_fwd(RasterVariant{}, T) ? 0 : 64;
+    const int def_bwd = !bd && few_bwd(RasterVariant{}, T) ? 0 : 32;
     out.fwd_ms = out.bwd_ms = 1e30f;
-    for (int fb : {32, 64, 128, 256})
+    for (int fb : {0, 32, 64, 128, 256})
       for (int mode = 0; mode < 4; mode++) {
+        if (fb == 0 && (def_fwd != 0 || mode > 0)) continue;
         RasterVariant rv;
         rv.fwd_batch = fb;
         rv.persistent = mode > 0;
@@ -1384,17 +1396,19 @@ RasterTune tune_raster(splat_ctx* ctx, const ProjBuffers& pb, const BinBuffers& 
                          counter);
         });
         out.candidates++;
-        if (rv.fwd_batch == def.fwd_batch && !rv.persistent) out.default_fwd_ms = ms;
+        if (rv.fwd_batch == def_fwd && !rv.persistent) out.default_fwd_ms = ms;
         if (ms < out.fwd_ms) {
           out.fwd_ms = ms;
           out.fwd = rv;
         }
       }
-    for (int bw : {16, 32})
+    for (int bw : {0, 16, 32})
       for (int mode = 0; mode < 8; mode++) {
+        if (bw == 0 && (ordered || def_bwd != 0 || mode > 0)) continue;
         RasterVariant rv;
-        rv.bwd_batch = bw;
-        rv.rows = mode < 4 || ordered;  // the ordered form walks per entry
+        // the ordered form has no such batches and walks per entry: the default is kept
+        rv.bwd_batch = ordered ? def_bwd : bw;
+        rv.rows = mode < 4 || ordered;
         if (ordered && mode >= 4) continue;
         rv.persistent = mode % 4 > 0;
         rv.per_cu = mode % 4 == 1 ? 2 : (mode % 4 == 2 ? 4 : 8);
@@ -1403,7 +1417,7 @@ RasterTune tune_raster(splat_ctx* ctx, const ProjBuffers& pb, const BinBuffers& 
                           slots, need_abs, rv, bd, counter);
         });
         out.candidates++;
-        if (rv.bwd_batch == def.bwd_batch && !rv.persistent && rv.rows) out.default_bwd_ms = ms;
+        if (rv.bwd_batch == def_bwd && !rv.persistent && rv.rows) out.default_bwd_ms = ms;
         if (ms < out.bwd_ms) {
           out.bwd_ms = ms;
           out.bwd = rv;
@@ -1419,6 +1433,11 @@ RasterTune tune_raster(splat_ctx* ctx, const ProjBuffers& pb, const BinBuffers& 
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   return out;
+}
+
+bool supported_batches(const splat_tune_result& shapes) {
+  const int f = shapes.fwd_batch, b = shapes.bwd_batch;
+  return (f == 0 || f == 32 || f == 64 || f == 128 || f == 256) && (b == 0 || b == 16 || b == 32);
 }
 
 void fill_tune_result(const RasterTune& t, splat_tune_result* out) {

@@ -942,10 +942,7 @@ int splat_trainer_pair_counts(splat_trainer* t, uint32_t view, const splat_step_
 int splat_trainer_set_shapes(splat_trainer* t, const splat_tune_result* shapes) {
   return tguard(t, [&] {
     SPLAT_REQUIRE(shapes, "null argument");
-    SPLAT_REQUIRE((shapes->fwd_batch == 32 || shapes->fwd_batch == 64 ||
-                   shapes->fwd_batch == 128 || shapes->fwd_batch == 256) &&
-                      (shapes->bwd_batch == 16 || shapes->bwd_batch == 32),
-                  "unsupported batch shape");
+    SPLAT_REQUIRE(supported_batches(*shapes), "unsupported batch shape");
     drain(t);
     t->fwd_shape.fwd_batch = shapes->fwd_batch;
     t->fwd_shape.persistent = shapes->fwd_persistent != 0;
