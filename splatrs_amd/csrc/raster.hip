@@ -814,7 +814,11 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
         le = next;
         next = my_list[min(t + 2, (uint32_t)B)];
         prepare();
-        const float out = now.template sums<false>(s, r2, bg_any, r0z, r0w, r1x, nullptr);
+        // the sums count if some lane evaluates the pair, as below: a factor of zero leaves a
+        // gradient that is not finite in them
+        const bool any = __builtin_amdgcn_ballot_w64(now.in) != 0;
+        const float sums = now.template sums<false>(s, r2, bg_any, r0z, r0w, r1x, nullptr);
+        const float out = any ? sums : 0.0f;
         if (has & writer) red[k16 * SS + my_red] = out;
       }
     } else {
