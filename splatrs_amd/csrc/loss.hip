@@ -28,7 +28,8 @@ constexpr int kHalo = 15;        // 5 pixels x 3 channels
 // rows before / this rule): 256x256 89 / 30, 400x304 90 / 37, 800x600 97 / 50, 1024x768
 // 103 / 67, 1297x840 104 / 84, 1600x1200 120 / 112, 1920x1080 121 / 122.
 constexpr unsigned kLossBlocks = 950;
-constexpr unsigned kMinLossRows = 2, kMaxLossRows = 64;
+// A lane adds its rows' loss terms one after the other in binary32, hence at most 32.
+constexpr unsigned kMinLossRows = 2, kMaxLossRows = 32;
 
 struct Taps {
   float k[11];

@@ -2,8 +2,8 @@
 pixel, one row or one column, chunks of two rows with a last chunk of one, strips that end
 inside a workgroup's 256 row elements, and images tall enough for long chunks.  The gradient
 is the reference's bit for bit whatever the split.  The loss value is a sum in an unspecified
-order: a lane sums at most 64 terms, a tree 256 lanes, the workgroups in binary64, so each mean
-is within (64 + 8 + 4) 2^-24 = 4.5e-6 of itself of the binary64 sum of the same terms; the
+order: a lane sums at most 32 terms, a tree 256 lanes, the workgroups in binary64, so each mean
+is within (32 + 8 + 4) 2^-24 = 2.6e-6 of itself of the binary64 sum of the same terms; the
 means are below 0.3 here (L1) and 1 (SSIM, weighed 0.2), so 2e-6 covers the loss."""
 import numpy as np
 import pytest
