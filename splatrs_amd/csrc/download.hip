@@ -115,8 +115,12 @@ void planes_to_host(splat_ctx* ctx, const HostRecords* arrays, size_t count) {
   for (size_t k = 0; k < count; k++) {
     const HostRecords& a = arrays[k];
     if (!a.out || a.n == 0) continue;
-    if (on_device(a.out)) {  // unified addresses: the kernel writes there itself
-      planes_to_aos(ctx, a.planes, a.n, a.stride, a.out);
+    if (on_device(a.out)) {  // the runtime checks the range and knows other devices' memory
+      DevBuf staging;
+      const size_t bytes = a.n * kParams * sizeof(float);
+      planes_to_aos(ctx, a.planes, a.n, a.stride, (float*)staging.reserve(bytes));
+      SPLAT_HIP(hipMemcpyAsync(a.out, staging.ptr, bytes, hipMemcpyDeviceToHost, ctx->stream));
+      SPLAT_HIP(hipStreamSynchronize(ctx->stream));
       continue;
     }
     for (size_t r = 0; r < a.n; r += kChunkRows)
