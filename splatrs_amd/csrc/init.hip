@@ -97,7 +97,7 @@ __global__ void __launch_bounds__(kKnnBlock) knn3_kernel(const float* __restrict
 // ---- larger clouds ----------------------------------------------------------------------
 
 constexpr uint32_t kKnnHalf = 8;  // Morton bits per axis and sort: two sorts, 16 bits per axis
-constexpr size_t kKnnBruteMax = 2048;  // see mean_nn_dist2_dev
+constexpr size_t kKnnBruteMax = 2560;  // see mean_nn_dist2_dev
 
 constexpr uint32_t kKnnQueries = 16;
 
@@ -121,14 +121,6 @@ __device__ __forceinline__ float lane_value(float v, uint32_t lane) {
   return bits2f((uint32_t)__builtin_amdgcn_readlane((int)f2bits(v), (int)lane));
 }
 
-// Floats as unsigned integers of the same order.
-__device__ __forceinline__ uint32_t ordered_bits(float f) {
-  const uint32_t u = f2bits(f);
-  return u ^ ((u >> 31) ? 0xffffffffu : 0x80000000u);
-}
-__device__ __forceinline__ float from_ordered(uint32_t u) {
-  return bits2f(u ^ ((u >> 31) ? 0x80000000u : 0xffffffffu));
-}
 __device__ __forceinline__ bool finite3(float x, float y, float z) {
   return fabsf(x) < INFINITY && fabsf(y) < INFINITY && fabsf(z) < INFINITY;
 }
@@ -143,40 +135,32 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
-// bounds[0..2] / [3..5]: least and greatest coordinates of the finite points, as ordered bits
-// (starting at all ones and zero).
-__global__ void __launch_bounds__(256) knn_bounds_kernel(const float* __restrict__ xyz, uint32_t n,
-                                                         uint32_t* __restrict__ bounds) {
-  float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const float p[3] = {xyz[3 * (size_t)i], xyz[3 * (size_t)i + 1], xyz[3 * (size_t)i + 2]};
-    if (!finite3(p[0], p[1], p[2])) continue;
+// bounds[0..2] / [3..5]: the range of most coordinates, from 256 points spread over the cloud:
+// all but the 4 least and the 4 greatest of an axis' finite ones.  (The least and greatest of
+// all points would put a scene into one cell if a single point lies far outside it.)
+constexpr uint32_t kKnnSamples = 256, kKnnTail = 4;
+__global__ void __launch_bounds__(kKnnSamples) knn_bounds_kernel(const float* __restrict__ xyz,
+                                                                 uint32_t n,
+                                                                 float* __restrict__ bounds) {
+  __shared__ float s[3][kKnnSamples];
+  const uint32_t k = threadIdx.x;
+  const size_t i = (size_t)((uint64_t)k * n / kKnnSamples);
+  const float p[3] = {xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2]};
+  const bool finite = finite3(p[0], p[1], p[2]);
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-      lo[c] = fminf(lo[c], p[c]);
-      hi[c] = fmaxf(hi[c], p[c]);
-    }
-  }
-  // one pair of atomics per block and axis: they meet in one line (one pair per wave of 512
-  // blocks took 141 us at 150k points, 13 us now)
-  __shared__ float slo[4], shi[4];
+  for (int c = 0; c < 3; c++) s[c][k] = finite ? p[c] : INFINITY;
+  const uint32_t count = (uint32_t)__syncthreads_count(finite ? 1 : 0);
+  const uint32_t tail = min(kKnnTail, count / 4);
+  if (k < 6 && count == 0) bounds[k] = 0.0f;
+  uint32_t rank[3] = {0, 0, 0};
+  for (uint32_t j = 0; j < kKnnSamples; j++)
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+      rank[c] += s[c][j] < p[c] || (s[c][j] == p[c] && j < k) ? 1u : 0u;
 #pragma unroll
   for (int c = 0; c < 3; c++) {
-    const float a = wave_min(lo[c]), b = wave_max(hi[c]);
-    __syncthreads();
-    if ((threadIdx.x & 63u) == 0) {
-      slo[threadIdx.x >> 6] = a;
-      shi[threadIdx.x >> 6] = b;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const float x = fminf(fminf(slo[0], slo[1]), fminf(slo[2], slo[3]));
-      const float y = fmaxf(fmaxf(shi[0], shi[1]), fmaxf(shi[2], shi[3]));
-      if (x <= y) {
-        atomicMin(&bounds[c], ordered_bits(x));
-        atomicMax(&bounds[3 + c], ordered_bits(y));
-      }
-    }
+    if (finite && rank[c] == tail) bounds[c] = p[c];
+    if (finite && rank[c] == count - 1 - tail) bounds[3 + c] = p[c];
   }
 }
 
@@ -191,7 +175,7 @@ __device__ __forceinline__ uint32_t spread3(uint32_t x) {
 // point order[k] (the upper half; points that are not finite behind all others).  16 bits per
 // axis keep the cells of a scene small next to points far outside it.
 __global__ void __launch_bounds__(256) knn_keys_kernel(const float* __restrict__ xyz, uint32_t n,
-                                                       const uint32_t* __restrict__ bounds,
+                                                       const float* __restrict__ bounds,
                                                        const uint32_t* __restrict__ order,
                                                        uint32_t* __restrict__ keys,
                                                        uint32_t* __restrict__ vals) {
@@ -204,10 +188,12 @@ __global__ void __launch_bounds__(256) knn_keys_kernel(const float* __restrict__
     code = 0;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      // any monotone cell will do: the boxes are taken from the points
-      const double lo = from_ordered(bounds[c]), span = (double)from_ordered(bounds[3 + c]) - lo;
-      const double at = span > 0 ? ((double)p[c] - lo) / span * (double)(1 << 2 * kKnnHalf) : 0.0;
-      const uint32_t cell = min((uint32_t)at, (1u << 2 * kKnnHalf) - 1u);
+      // any monotone cell will do: the boxes are taken from the points.  The cells cover the
+      // bounds and a quarter of their span on either side; points beyond share the last cells.
+      const double lo = bounds[c], span = (double)bounds[3 + c] - lo;
+      const double at = span > 0 ? ((double)p[c] - lo) / span + 0.25 : 0.0;
+      const double top = (double)((1u << 2 * kKnnHalf) - 1u);
+      const uint32_t cell = (uint32_t)fmin(fmax(at * (1.0 / 1.5) * (top + 1.0), 0.0), top);
       code |= spread3(order ? cell >> kKnnHalf : cell & ((1u << kKnnHalf) - 1u)) << c;
     }
   }
@@ -275,9 +261,10 @@ __device__ __forceinline__ double box_dist2(float4 alo, float4 ahi, float4 blo, 
 // queries and the largest of their bounds; then by each query); at the end the four lanes' lists
 // are merged.  A candidate's distance is first taken in binary32, with room for its rounding, and
 // in binary64 only where that leaves it possible.  Bound by the latency of a block visit (points
-// loaded while the previous block is looked at): 163 us at 150k points (a lane per query and 64
-// queries per wave, all distances in binary64: above 500 us, its last waves those of the points
-// outside the scene).
+// loaded while the previous block is looked at): 294 us for 150k points
+// on twenty ellipsoids with 2 % in a box of six times their size (381 us with cells over all
+// points' range; a lane per query and 64 queries per wave, all distances in binary64, took three
+// times as long, its last waves those of the points far out).
 __global__ void __launch_bounds__(64) knn_query_kernel(const float* __restrict__ xyz, uint32_t n,
                                                        uint32_t nb, uint32_t ns,
                                                        const float4* __restrict__ pts,
@@ -422,11 +409,12 @@ __global__ void __launch_bounds__(64) knn_query_kernel(const float* __restrict__
 }  // namespace
 
 // Brute force costs a chain of n distances per lane, 90 us per 1000 points, and n^2 once the chip
-// is full; the boxes cost 23 small launches (the Morton order is 140 us of them) and then about
-// n log n.  A whole call in us, brute force / boxes, points of a shell with 2 % outside it:
-// 1100: 151 / 212, 2000: 244 / 250, 4000: 430 / 345, 16000: 1524 / 435, 50000: 4194 / 404,
-// 150000: 14231 / 623.  150000 points all the same: 14085 / 3126; one of them 10^7 scene radii
-// away, so that all others share a cell: 14231 / 14348.
+// is full; the boxes cost 21 small launches (the Morton order is 140 us of them) and then about
+// n log n.  A whole call in us, brute force / boxes, points in a cube: 2049 246 / 267, 2500
+// 291 / 281, 3000 336 / 303, 5000 521 / 364, 16000 1402 / 357, 50000 4165 / 412, 150000
+// 14090 / 645; all points the same: 2500 251 / 252, 150000 13944 / 3071; on a shell with 2 % up to
+// twenty radii out: 150000 14136 / 880; in a cube with one point 10^7 away: 150000 14130 / 628
+// (cells over all points' range: 14127).
 void mean_nn_dist2_dev(splat_ctx* ctx, const float* xyz, size_t n, double* out) {
   if (n <= kKnnBruteMax) {
     launch(ctx, "knn3", knn3_kernel, dim3(blocks_for(n, kKnnBlock)), dim3(kKnnBlock), 0, xyz,
@@ -435,7 +423,7 @@ void mean_nn_dist2_dev(splat_ctx* ctx, const float* xyz, size_t n, double* out) 
   }
   SPLAT_REQUIRE(n < 0xffffffffull - 64, "too many points");
   const unsigned nb = blocks_for(n, 64), ns = blocks_for(nb, 64);
-  uint32_t* bounds = ctx->buf<uint32_t>("knn_bounds", 6);
+  float* bounds = ctx->buf<float>("knn_bounds", 6);
   uint32_t* k0 = ctx->buf<uint32_t>("knn_k0", n);
   uint32_t* v0 = ctx->buf<uint32_t>("knn_v0", n);
   uint32_t* k1 = ctx->buf<uint32_t>("knn_k1", n);
@@ -446,19 +434,17 @@ void mean_nn_dist2_dev(splat_ctx* ctx, const float* xyz, size_t n, double* out) 
   float4* pts = ctx->buf<float4>("knn_pts", n);
   float4* boxes = ctx->buf<float4>("knn_boxes", 2 * (size_t)nb + 2 * (size_t)ns);
   float4 *lo = boxes, *hi = lo + nb, *slo = hi + nb, *shi = slo + ns;
-  fill_u32(ctx, bounds, 3, 0xffffffffu);
-  fill_u32(ctx, bounds + 3, 3, 0u);
-  launch(ctx, "knn_bounds", knn_bounds_kernel, dim3(std::min(blocks_for(n, 256), 128u)), dim3(256),
-         0, xyz, (uint32_t)n, bounds);
+  launch(ctx, "knn_bounds", knn_bounds_kernel, dim3(1), dim3(kKnnSamples), 0, xyz, (uint32_t)n,
+         bounds);
   launch(ctx, "knn_keys", knn_keys_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, xyz,
-         (uint32_t)n, (const uint32_t*)bounds, (const uint32_t*)nullptr, k0, v0);
+         (uint32_t)n, (const float*)bounds, (const uint32_t*)nullptr, k0, v0);
   if (radix_sort_pairs(ctx, k0, v0, k1, v1, n, (uint32_t)n, nullptr, 3 * kKnnHalf, counts, sums,
                        nullptr)) {
     std::swap(k0, k1);
     std::swap(v0, v1);
   }
   launch(ctx, "knn_keys", knn_keys_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, xyz,
-         (uint32_t)n, (const uint32_t*)bounds, (const uint32_t*)v0, k0, (uint32_t*)nullptr);
+         (uint32_t)n, (const float*)bounds, (const uint32_t*)v0, k0, (uint32_t*)nullptr);
   const int c = radix_sort_pairs(ctx, k0, v0, k1, v1, n, (uint32_t)n, nullptr, 3 * kKnnHalf + 1,
                                  counts, sums, nullptr);
   launch(ctx, "knn_blocks", knn_blocks_kernel, dim3(nb), dim3(64), 0, xyz, (uint32_t)n,
