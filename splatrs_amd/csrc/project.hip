@@ -742,8 +742,9 @@ __device__ __forceinline__ void adam_groups(float* __restrict__ params, float* _
 // R rows and THREADS lanes per workgroup: 128 and 128 stream large models.  A model of up to
 // kGradAdamSmall rows gets too few such workgroups to fill the chip, and each of them takes its
 // 1888 float4 groups in four rounds of 16 loads per lane; with 64 rows and 256 lanes (the first
-// 64 run the projection backward) there are twice as many workgroups and one round: 31 -> 20 us
-// at 10k rows, 53 -> 44 at 61k (300k: 109 -> 143, 1M: 287 -> 387, which keep the large form).
+// 64 run the projection backward) there are twice as many workgroups and one round.  In us,
+// small form / large, on scenes of 0.15 to 0.27 Gaussians per pixel: 10k rows 23 / 40, 26k
+// 25 / 39, 46k 30 / 43, 61k 45 / 45, 77k 49 / 51, 104k 64 / 54, 207k 107 / 91, 311k 154 / 118.
 constexpr uint32_t kGradAdamRows = 128, kGradAdamRowsSmall = 64, kGradAdamSmall = 1u << 16;
 constexpr uint32_t kGradWords = 11 + 16 + 3;  // LDS words per row: planes 0-10, basis, dc
 

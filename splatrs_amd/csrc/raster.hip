@@ -20,14 +20,24 @@ namespace {
 
 // Launches of one view with few tiles in the default shape: each wave's own latency bounds them,
 // and registers and LDS are free.  The FEW kernels evaluate a step's pair beside the previous
-// step's state update, without a branch, and take larger batches (fewer barriers).  Forward, in
-// us, FEW with 256-entry batches against 64-entry ones: 256 tiles 39 / 53, 1271 tiles 50 / 57,
-// 4293 tiles 192 / 199, 8160 tiles 185 / 179.  Backward, FEW with 64-entry batches (45 KB of
-// LDS: three workgroups per compute unit) against 32: 256 tiles 97 / 118, 1271 tiles 115 /
-// 140, 4293 tiles 502 / 363; FEW with 32-entry batches lies between at all four sizes.
-constexpr unsigned kFewTilesFwd = 6144;
+// step's state update, without a branch, and take larger batches (fewer barriers): the forward
+// 256 entries instead of 64, the backward 64 (45 KB of LDS: three workgroups per compute unit)
+// instead of 32.  In us, FEW / otherwise, on a light scene (0.15 Gaussians per pixel, in a box)
+// and a dense one (0.27, on surfaces):
+//   tiles    forward                     backward
+//    256     43 /  57   127 / 150        103 / 128   252 / 287
+//    900     47 /  61   143 / 167        112 / 137   282 / 322
+//   1600     50 /  63   169 / 190        116 / 140   324 / 358
+//   2000     46 /  56   153 / 171        104 / 123   288 / 321
+//   2700     55 /  56   161 / 175        136 / 118   297 / 335
+//   4346     91 /  91   184 / 188        248 / 188   495 / 367
+//   5400    112 / 112   225 / 218        315 / 233   611 / 425
+// The lines lie where neither scene is slower.  (The general forward with 256 entries is between
+// the two up to 2000 tiles and below both from 2700 on, 159 at 4346 on the dense scene; tuning
+// finds it.)
+constexpr unsigned kFewTilesFwd = 4608;
 constexpr unsigned kFewTilesBwd = 1536;
-constexpr unsigned kFewTilesOrd = 768;  // ordered backward, see raster_bwd_ordered_kernel
+constexpr unsigned kFewTilesOrd = 768;  // see raster_bwd_ordered_kernel
 constexpr int kOrdBatch = 32;      // entries staged per batch (ordered backward)
 
 struct TileInfo {
@@ -240,8 +250,8 @@ struct FwdPair {
 // instructions in each: the four 16-lane rows of a wave walk lists of their own (against one
 // walk of the entries that reach the wave's 8x8 block: about a fifth fewer steps), and a list
 // word carries the pixels of the row's sub-block that the entry's rectangle holds, one AND
-// instead of four comparisons.  At 1M Gaussians, 1920x1080: 226 -> 175 us; 10k Gaussians,
-// 256x256: 82 -> 63 us.
+// instead of four comparisons.  10k Gaussians, 256x256: 82 -> 63 us; with 256 entries per batch
+// and records prefetched too, 1M Gaussians, 1920x1080: 227 -> 190 us.
 // B: entries per LDS batch; BATCH: tiles of many views (BatchDev); PERSIST: a fixed grid
 // that takes tiles from `counter` until `num_tiles` are done; COUNT: also count pairs
 // into `pairs` (PairCounter); FEW: for launches with few tiles (kFewTilesFwd).
@@ -639,8 +649,8 @@ __device__ __forceinline__ PixBack pixel_back(const TileGeom& tg, uint32_t i, ui
 // summed in a fixed order.  Bound by VALU issue (about 100 instructions per walk step).  Of
 // the LDS partials only those that svisit names are written and read: clearing all 16 rows of
 // every entry and summing them took as many instructions as a fifth of the walk.  With that,
-// the list words (as in the forward) and the row sums in one block: 1M Gaussians, 1920x1080,
-// 471 -> 400 us; 10k, 256x256, 139 -> 123 us.
+// the list words (as in the forward) and the row sums in one block: 10k Gaussians, 256x256,
+// 139 -> 123 us; with records prefetched too, 1M Gaussians, 1920x1080: 471 -> 428 us.
 // ABS: also accumulate the AbsGS slots (9, 10).  B: entries per LDS batch.  ROWS: every
 // 16-lane row walks its own entry list; otherwise the wave walks the entries that reach any
 // of its rows (the same sums either way).  COUNT: also count pairs into `pairs`
@@ -894,7 +904,7 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
 // The ordered backward: an entry's per-pixel terms are staged in LDS and summed one by one
 // in row-major order.  Only the pixels of the entry's rectangle have terms (the others are
 // exact zeros, which a sum that starts at +0 does not see), so the staging is packed: the
-// entries of a group, as many as fit kOrdTerms pixels, lie one after the other, and a lane
+// entries of a group, as many as fit kTerms pixels, lie one after the other, and a lane
 // sums one slot of one entry over the entry's own pixels.  Only the waves whose 8x8 block the
 // rectangle reaches evaluate it.
 //
@@ -905,10 +915,12 @@ __global__ void __launch_bounds__(256) raster_bwd_kernel(
 // workgroups, walk and sums take turns and the staging is kept small (two full tiles).  In us,
 // FEW / otherwise / all 256 pixels of 8 entries staged at a time, as it was: 130 tiles of a
 // grown model (most entries cover their tiles) 511 / 680 / 1279, 256 tiles 177 / 229 / 403,
-// 1271 tiles 337 / 250 / 767, 4293 tiles 2060 / 875 / 4526, 8160 tiles 2401 / 750 / 5785.  (The
-// slots' rows lie four words apart modulo the LDS banks and are read 16 bytes at a time, the
-// next ones beside the additions; in step and one word at a time it was 940 at 130 tiles and
-// 1217 at 8160.)
+// 4293 tiles 2060 / 875 / 4526, 8160 tiles 2401 / 750 / 5785.  FEW / otherwise on the scenes of
+// kFewTilesFwd: 675 tiles 187 / 244 and 593 / 814, 900 tiles 204 / 262 and 507 / 700, 1120 tiles
+// 245 / 246 and 543 / 756, 1271 tiles 262 / 206 and 497 / 696, 1600 tiles 336 / 269 and 630 / 872:
+// the line lies where neither is slower.  (The slots' rows lie four words apart modulo the LDS
+// banks and are read 16 bytes at a time, the next ones beside the additions; in step and one word
+// at a time it was 940 at 130 tiles and 1217 at 8160.)
 template <bool ABS, bool BATCH, bool PERSIST, bool FEW>
 __global__ void __launch_bounds__(FEW ? 320 : 256) raster_bwd_ordered_kernel(
     const float4* __restrict__ rec, const uint32_t* __restrict__ tile_start,
