@@ -22,8 +22,8 @@ constexpr int kStrip = 256;
 constexpr int kHalo = 15;        // 5 pixels x 3 channels
 
 // Rows per workgroup.  A workgroup of r rows blurs r + 10 (the halo), one after the other, and
-// three workgroups share a compute unit, so large images want long chunks and small images
-// enough workgroups.  The shortest chunk that keeps a launch to kLossBlocks workgroups was
+// kLossBlocks makes three to four workgroups per compute unit (their registers would let four or
+// five fit), so large images want long chunks and small images enough workgroups.  The shortest chunk that keeps a launch to kLossBlocks workgroups was
 // within 5% of the best of 2..64 rows at every size measured (both passes, in us, fixed 32
 // rows before / this rule): 256x256 89 / 30, 400x304 90 / 37, 800x600 97 / 50, 1024x768
 // 103 / 67, 1297x840 104 / 84, 1600x1200 120 / 112, 1920x1080 121 / 122.
